@@ -1,0 +1,10 @@
+// ifos_order5.hip -- time-loop kernels of FDORDER 10.
+#include "ifos_step_kernels.h"
+
+namespace ifos {
+
+template void vel_n<5>(const StepArgs &a, const StepArgs *da, const LaunchShape &ls, int k, hipStream_t s);
+template void str_n<5>(const StepArgs &a, const StepArgs *da, const LaunchShape &ls, int k, hipStream_t s);
+template void fused_n<5>(const StepArgs &a, const StepArgs *da, const LaunchShape &ls, int k, hipStream_t s);
+
+}  // namespace ifos
