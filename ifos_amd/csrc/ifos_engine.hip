@@ -150,12 +150,12 @@ struct ifos_engine {
     double *trace_sums = nullptr;  // l2, en [2][cap_tr]
     std::vector<double> shot_misfit;  // l2, en per shot of the last residual
 
-    // per-slot, per-tile point lists (sources, receivers) for the step kernels
+    // sources and receivers by cell and tile for the step kernels (PointMap)
     int nbx = 0, nby = 0;
-    int *tiles = nullptr;
+    int *tiles = nullptr;    // start and next of the sources, then of the receivers, then the map entries
     size_t tiles_cap = 0;
-    int off_src_start = 0, off_src_idx = 0, off_rec_start = 0, off_rec_idx = 0;
-    int off_srcx_start = 0, off_srcx_idx = 0, off_recx_start = 0, off_recx_idx = 0;  // tile + rim lists
+    int off_src_start = 0, off_src_next = 0, off_rec_start = 0, off_rec_next = 0;
+    int *point_map = nullptr;  // [2][slots][plane]: sources, receivers
     LaunchShape shape;
     // energy preconditioner (src/eprecond.c, src/eprecond1.c): Ws and Wr per
     // slot, the 1/We sum over shots, the mode-3 geometric factor
@@ -358,6 +358,7 @@ static int engine_create(const ifos_config *cfg, int device, int slots, ifos_eng
     if (dmalloc(&E->explosive, sizeof(int) * slots) != hipSuccess) return fail(-3);
     hipMemsetAsync(E->explosive, 0, sizeof(int) * slots, E->stream);
     if (dmalloc(&E->dargs, sizeof(StepArgs) * 4) != hipSuccess) return fail(-3);
+    if (dmalloc(&E->point_map, sizeof(int) * 2 * E->plane * slots) != hipSuccess) return fail(-3);
     if (hipStreamSynchronize(E->stream) != hipSuccess) {
         ifos_set_error("engine set-up failed on the device");
         return fail(-1);
@@ -396,7 +397,7 @@ extern "C" void ifos_engine_destroy(ifos_engine *E)
     dfree(E->wbuf); dfree(E->wbuf64); dfree(E->we_sum); dfree(E->ep_geom); dfree(E->we_max); dfree(E->red);
     dfree(E->tap_m); dfree(E->tap_ij); dfree(E->tap_lohi); dfree(E->tfbuf);
     dfree(E->src_i); dfree(E->src_d); dfree(E->sig); dfree(E->rec_i); dfree(E->seis);
-    dfree(E->trace_sums); dfree(E->snap); dfree(E->tiles);
+    dfree(E->trace_sums); dfree(E->snap); dfree(E->tiles); dfree(E->point_map);
     if (E->stream) hipStreamDestroy(E->stream);
     ifos_free_materials(&E->mat);
     delete E;
@@ -468,6 +469,13 @@ static void filter_traces(ifos_engine *E, float *d, int ntr, bool apply)
     f.nhigh = E->filt_nhigh;
     memcpy(f.c, E->filt_c, sizeof f.c);
     launch_time_filter(f, E->stream);
+}
+
+// enter the first point of each cell that holds points
+__global__ void k_point_map(int *map_, const long *at_, const int *first_, int n)
+{
+    const int q = blockIdx.x * blockDim.x + threadIdx.x;
+    if (q < n) gmem(map_)[gmem(at_)[q]] = gmem(first_)[q];
 }
 
 // shots of the slots: slot s has nsrc[s] sources (rows of srcpos, all
@@ -570,79 +578,48 @@ extern "C" int ifos_engine_set_shots(ifos_engine *E, int nshots, const int *nsrc
         HIP_TRY(hipMemcpyAsync(E->rec_i, ri.data(), sizeof(int) * ri.size(), hipMemcpyHostToDevice, E->stream));
         HIP_TRY(hipStreamSynchronize(E->stream));
     }
-    // bucket each slot's sources and receivers by 64x8 tile, keeping their order
+    // sources and receivers by tile (running counts) and by cell (the first
+    // point of each cell, and the chain of those at the same one, in order)
     const int nblk = E->nbx * E->nby;
-    auto bucket = [&](const std::vector<int> &off, auto x_of, auto y_of, std::vector<int> &start,
-                      std::vector<int> &idx) {
-        const int n = off[nshots];
-        start.assign((size_t)nshots * (nblk + 1), 0);
-        idx.assign(n > 0 ? n : 1, 0);
-        int pos = 0;
-        for (int k = 0; k < nshots; k++) {
-            int *st = start.data() + (size_t)k * (nblk + 1);
-            std::vector<int> tile(off[k + 1] - off[k]);
-            for (int q = off[k]; q < off[k + 1]; q++) {
-                tile[q - off[k]] = ((y_of(q) - 1) / kTileY) * E->nbx + (x_of(q) - 1) / kTileX;
-                st[tile[q - off[k]] + 1]++;
-            }
-            st[0] = pos;
-            for (int b = 0; b < nblk; b++) st[b + 1] += st[b];
-            std::vector<int> fill(st, st + nblk);
-            for (int q = off[k]; q < off[k + 1]; q++) idx[fill[tile[q - off[k]]]++] = q;
-            pos = st[nblk];
-        }
-    };
-    std::vector<int> s_start, s_idx, r_start, r_idx;
-    bucket(so, [&](int q) { return (int)srcpos[(size_t)q * IFOS_SRC_STRIDE]; },
-           [&](int q) { return (int)srcpos[(size_t)q * IFOS_SRC_STRIDE + 1]; }, s_start, s_idx);
-    bucket(to, [&](int q) { return recpos[2 * q]; }, [&](int q) { return recpos[2 * q + 1]; }, r_start, r_idx);
-    // the same per tile for the tile and its N-cell rim (k_fused_step): a
-    // point is listed for every tile whose rim reaches it, in point order
-    auto bucket_rim = [&](const std::vector<int> &off, auto x_of, auto y_of, std::vector<int> &start,
-                          std::vector<int> &idx) {
-        const int R = E->N;
-        start.assign((size_t)nshots * (nblk + 1), 0);
-        std::vector<std::vector<int>> per(nblk);
-        idx.clear();
-        for (int k = 0; k < nshots; k++) {
-            for (auto &v : per) v.clear();
-            for (int q = off[k]; q < off[k + 1]; q++) {
-                const int x = x_of(q), y = y_of(q);
-                const int bx0 = std::max(0, (x - 1 - R) / kTileX), bx1 = std::min(E->nbx - 1, (x - 1 + R) / kTileX);
-                const int by0 = std::max(0, (y - 1 - R) / kTileY), by1 = std::min(E->nby - 1, (y - 1 + R) / kTileY);
-                for (int by = by0; by <= by1; by++)
-                    for (int bx = bx0; bx <= bx1; bx++) per[by * E->nbx + bx].push_back(q);
-            }
-            int *st = start.data() + (size_t)k * (nblk + 1);
-            st[0] = (int)idx.size();
-            for (int b = 0; b < nblk; b++) {
-                idx.insert(idx.end(), per[b].begin(), per[b].end());
-                st[b + 1] = (int)idx.size();
-            }
-        }
-        if (idx.empty()) idx.push_back(0);
-    };
-    std::vector<int> sx_start, sx_idx, rx_start, rx_idx;
-    bucket_rim(so, [&](int q) { return (int)srcpos[(size_t)q * IFOS_SRC_STRIDE]; },
-               [&](int q) { return (int)srcpos[(size_t)q * IFOS_SRC_STRIDE + 1]; }, sx_start, sx_idx);
-    bucket_rim(to, [&](int q) { return recpos[2 * q]; }, [&](int q) { return recpos[2 * q + 1]; }, rx_start, rx_idx);
     std::vector<int> blob;
-    E->off_src_start = 0;
-    blob.insert(blob.end(), s_start.begin(), s_start.end());
-    E->off_src_idx = (int)blob.size();
-    blob.insert(blob.end(), s_idx.begin(), s_idx.end());
-    E->off_rec_start = (int)blob.size();
-    blob.insert(blob.end(), r_start.begin(), r_start.end());
-    E->off_rec_idx = (int)blob.size();
-    blob.insert(blob.end(), r_idx.begin(), r_idx.end());
-    E->off_srcx_start = (int)blob.size();
-    blob.insert(blob.end(), sx_start.begin(), sx_start.end());
-    E->off_srcx_idx = (int)blob.size();
-    blob.insert(blob.end(), sx_idx.begin(), sx_idx.end());
-    E->off_recx_start = (int)blob.size();
-    blob.insert(blob.end(), rx_start.begin(), rx_start.end());
-    E->off_recx_idx = (int)blob.size();
-    blob.insert(blob.end(), rx_idx.begin(), rx_idx.end());
+    std::vector<long> at;   // cell of each map entry, receivers offset by all slots' planes
+    std::vector<int> first;
+    auto place = [&](const std::vector<int> &off, long base, auto x_of, auto y_of, int &off_start, int &off_next) {
+        off_start = (int)blob.size();
+        blob.resize(blob.size() + (size_t)nshots * (nblk + 1), 0);
+        int *start = blob.data() + off_start;
+        std::vector<std::pair<long, int>> cell(off[nshots]);
+        for (int k = 0; k < nshots; k++) {
+            int *st = start + (size_t)k * (nblk + 1);
+            for (int q = off[k]; q < off[k + 1]; q++) {
+                const int x = x_of(q) - 1, y = y_of(q) - 1;
+                st[(y / kTileY) * E->nbx + x / kTileX + 1]++;
+                cell[q] = {base + (long)k * E->plane + (long)y * c.NX + x, q};
+            }
+            for (int b = 0; b < nblk; b++) st[b + 1] += st[b];
+        }
+        std::sort(cell.begin(), cell.end());
+        off_next = (int)blob.size();
+        blob.resize(blob.size() + std::max(1, off[nshots]), -1);
+        int *next = blob.data() + off_next;
+        for (size_t q = 0; q < cell.size(); q++)
+            if (q && cell[q].first == cell[q - 1].first) {
+                next[cell[q - 1].second] = cell[q].second;
+            } else {
+                at.push_back(cell[q].first);
+                first.push_back(cell[q].second);
+            }
+    };
+    const long planes = E->plane * E->slots;
+    place(so, 0, [&](int q) { return (int)srcpos[(size_t)q * IFOS_SRC_STRIDE]; },
+          [&](int q) { return (int)srcpos[(size_t)q * IFOS_SRC_STRIDE + 1]; }, E->off_src_start, E->off_src_next);
+    place(to, planes, [&](int q) { return recpos[2 * q]; }, [&](int q) { return recpos[2 * q + 1]; },
+          E->off_rec_start, E->off_rec_next);
+    const int npoint = (int)first.size();
+    const size_t off_first = blob.size(), off_at = (off_first + npoint + 1) / 2 * 2;  // 8-byte aligned
+    blob.resize(off_at + 2 * (size_t)npoint);
+    std::copy(first.begin(), first.end(), blob.begin() + off_first);
+    memcpy(blob.data() + off_at, at.data(), sizeof(long) * npoint);
     if (blob.size() > E->tiles_cap) {
         dfree(E->tiles);
         E->tiles = nullptr;
@@ -651,6 +628,12 @@ extern "C" int ifos_engine_set_shots(ifos_engine *E, int nshots, const int *nsrc
         drop_graphs(E);
     }
     HIP_TRY(hipMemcpyAsync(E->tiles, blob.data(), sizeof(int) * blob.size(), hipMemcpyHostToDevice, E->stream));
+    HIP_TRY(hipMemsetAsync(E->point_map, 0xFF, sizeof(int) * 2 * (size_t)planes, E->stream));
+    if (npoint) {
+        hipLaunchKernelGGL(k_point_map, dim3((npoint + 255) / 256), dim3(256), 0, E->stream, E->point_map,
+                           (const long *)(E->tiles + off_at), E->tiles + off_first, npoint);
+        HIP_TRY(hipGetLastError());
+    }
     HIP_TRY(hipStreamSynchronize(E->stream));
     return 0;
 }
@@ -731,23 +714,21 @@ static StepArgs step_args(ifos_engine *E, int sw, bool snapshots)
     a.vx2 = E->vx2; a.vy2 = E->vy2; a.sxx2 = E->sxx2; a.syy2 = E->syy2; a.sxy2 = E->sxy2;
     a.psi2_sxx_x = E->psi2_sxx_x; a.psi2_sxy_x = E->psi2_sxy_x; a.psi2_syy_y = E->psi2_syy_y;
     a.psi2_sxy_y = E->psi2_sxy_y;
-    TileList src;
-    src.start = E->tiles + E->off_src_start; src.idx = E->tiles + E->off_src_idx;
-    src.ix = E->src_i; src.iy = E->src_i + E->cap_src; src.type = E->src_i + 2 * E->cap_src;
+    PointMap src;
+    src.start = E->tiles + E->off_src_start; src.next = E->tiles + E->off_src_next;
+    src.map = E->point_map;
+    src.type = E->src_i + 2 * E->cap_src;
     src.sin_azi = E->src_d; src.cos_azi = E->src_d + E->cap_src;
     src.sig = E->sig; src.sig1 = E->sig;
-    TileList rec;
-    rec.start = E->tiles + E->off_rec_start; rec.idx = E->tiles + E->off_rec_idx;
-    rec.ix = E->rec_i; rec.iy = E->rec_i + E->cap_tr; rec.type = nullptr;
+    PointMap rec;
+    rec.start = E->tiles + E->off_rec_start; rec.next = E->tiles + E->off_rec_next;
+    rec.map = E->point_map + E->plane * E->slots;
+    rec.type = nullptr;
     rec.sin_azi = rec.cos_azi = nullptr;
     rec.sig = seis_buf(E, 2); rec.sig1 = seis_buf(E, 3);  // adjoint sources
     a.inj = sw == 0 ? src : rec;
     a.exp = src;
     a.rec = rec;
-    TileList srcx = src, recx = rec;
-    srcx.start = E->tiles + E->off_srcx_start; srcx.idx = E->tiles + E->off_srcx_idx;
-    recx.start = E->tiles + E->off_recx_start; recx.idx = E->tiles + E->off_recx_idx;
-    a.injx = sw == 0 ? srcx : recx;
     a.explosive = E->explosive;
     a.snap_prec = E->snap_prec;
     if (snapshots || sw == 1) {
@@ -1488,6 +1469,7 @@ extern "C" size_t ifos_engine_bytes(const ifos_config *c, int slots, int snap_pr
     b += sizeof(float) * field * (size_t)(15 + 3 * c->L);                 // materials
     b += sizeof(float) * plane * (11 + 3 * (size_t)slots);                // interior + correlation
     b += sizeof(float) * (size_t)(7 * c->NY * fw2 + 6 * fw2 * c->NX) * slots;  // CPML memory
+    b += sizeof(int) * 2 * plane * slots;                                 // cells of sources and receivers
     b += sizeof(float) * (size_t)6 * ntr_total * c->NT;                   // seismograms etc.
     b += (sizeof(float) * c->NT + 3 * sizeof(int) + 2 * sizeof(double)) * (size_t)nsrc_total;
     b += (3 * sizeof(int) + 2 * sizeof(double)) * (size_t)ntr_total;

@@ -14,9 +14,8 @@
 // Each launch advances every active shot slot (one shot of the same model per
 // slot).  Work items are (tile, group of spb slots) pairs; a thread owns one
 // cell of a 64x8 tile and loops over the slots of its group, loading the
-// cell's materials once.  Point sources and receivers are bucketed per slot
-// and tile on the host (CSR lists in source order), so a thread only scans
-// the few points of its own tile.  The free surface needs the new
+// cell's materials once.  Point sources and receivers are looked up by cell
+// (PointMap), in tiles that hold any.  The free surface needs the new
 // stresses of rows 2..N+1 of its column: tiles are 8 rows high and N <= 6, so
 // the top tile row holds them; they are exchanged through LDS after a barrier.
 // The arithmetic is the per-cell code of ifos_cellmath.h, bit-identical to
@@ -62,10 +61,7 @@ __device__ __forceinline__ void vel_cell(const StepArgs &a, int s, int blk, int 
         vx0 = vxs[c];
         vy0 = vys[c];
     }
-    // bounds of this tile's point-force / residual list, loaded behind the
-    // stencil loads so that their latency overlaps them
-    const int so = __builtin_amdgcn_readfirstlane(s * (a.nbx * a.nby + 1) + blk);  // uniform
-    const int q0 = cmem(a.inj.start)[so], q1 = cmem(a.inj.start)[so + 1];
+    const int p0 = live ? first_point(a, a.inj, s, e, tile_has(a.inj, s, a.nbx * a.nby, blk)) : -1;
     if (flags & kForward) {
         if (flags & kSnapStep) {
             const float val[2] = {vel_rate(rip, sxx_x + sxy_y, g.DH), vel_rate(rjp, sxy_x + syy_y, g.DH)};
@@ -83,29 +79,8 @@ __device__ __forceinline__ void vel_cell(const StepArgs &a, int s, int blk, int 
     float vx = vel_new(vx0, g.DT, rip, sxx_x + sxy_y, g.DH);
     float vy = vel_new(vy0, g.DT, rjp, sxy_x + syy_y, g.DH);
 
-    // point forces (forward) / residual injection (adjoint) of this tile, in order
-    // the point index is the same for the whole wave: the list, position and
-    // signal reads are scalar loads, the cell match is per lane
-    for (int q = q0; q < q1; q++) {
-        const int l = cmem(a.inj.idx)[q];
-        const int px = cmem(a.inj.ix)[l], py = cmem(a.inj.iy)[l];
-        const float s0 = cmem(a.inj.sig)[(long)l * a.NT + nt - 1];
-        const float s1 = cmem(a.inj.sig1)[(long)l * a.NT + nt - 1];
-        if (px != i || py != j) continue;
-        if (a.sw == 0) {
-            const int type = cmem(a.inj.type)[l];
-            if (type == 2) vx += (g.DT * rip * s1) / (g.DH * g.DH);
-            if (type == 3) vy += (g.DT * rjp * s1) / (g.DH * g.DH);
-            if (type == 4) {
-                vx += (g.DT * rip * cmem(a.inj.sin_azi)[l] * s0) / (g.DH * g.DH);
-                vy += (g.DT * rjp * cmem(a.inj.cos_azi)[l] * s0) / (g.DH * g.DH);
-            }
-        } else {
-            if (a.ADJOINT_TYPE == 1) { vx += s0; vy += s1; }
-            if (a.ADJOINT_TYPE == 2) vy += s1;
-            if (a.ADJOINT_TYPE == 3) vx += s0;
-        }
-    }
+    // point forces (forward) / residual injection (adjoint) at this cell, in order
+    for (int l = p0; l >= 0; l = gmem(a.inj.next)[l]) inject(a, l, nt, rip, rjp, vx, vy);
     vxs[c] = vx;
     vys[c] = vy;
     if (g.BOUNDARY) wrap_pair<N>(g, vys, vxs, c, i, vy, vx);
@@ -154,8 +129,7 @@ __device__ __forceinline__ void vel_rows_with(const StepArgs &a, int s, int blk,
                 cpml_velocity(g, j + r, i, a.psi_sxx_x + po, a.psi_sxy_x + po, a.psi_syy_y + po, a.psi_sxy_y + po,
                               sxx_x[r], sxy_x[r], sxy_y[r], syy_y[r]);
     }
-    const int so = __builtin_amdgcn_readfirstlane(s * (a.nbx * a.nby + 1) + blk);  // uniform
-    const int q0 = cmem(a.inj.start)[so], q1 = cmem(a.inj.start)[so + 1];
+    const bool points = tile_has(a.inj, s, a.nbx * a.nby, blk);
     if (flags & kForward) {
         if (flags & kSnapStep) {
             float val[R][2];
@@ -188,31 +162,13 @@ __device__ __forceinline__ void vel_rows_with(const StepArgs &a, int s, int blk,
         vx[r] = vel_new(vx0[r], g.DT, rip[r], sxx_x[r] + sxy_y[r], g.DH);
         vy[r] = vel_new(vy0[r], g.DT, rjp[r], sxy_x[r] + syy_y[r], g.DH);
     }
-    // point forces / residual injection of this tile, in list order; a point
-    // lands on at most one of the R cells
-    for (int q = q0; q < q1; q++) {
-        const int l = cmem(a.inj.idx)[q];
-        const int px = cmem(a.inj.ix)[l], py = cmem(a.inj.iy)[l];
-        const float s0 = cmem(a.inj.sig)[(long)l * a.NT + nt - 1];
-        const float s1 = cmem(a.inj.sig1)[(long)l * a.NT + nt - 1];
-        if (px != i || py < j || py >= j + R) continue;
+    // point forces / residual injection of these cells, in order
+    if (points) {
 #pragma unroll
-        for (int r = 0; r < R; r++) {
-            if (py != j + r) continue;
-            if (a.sw == 0) {
-                const int type = cmem(a.inj.type)[l];
-                if (type == 2) vx[r] += (g.DT * rip[r] * s1) / (g.DH * g.DH);
-                if (type == 3) vy[r] += (g.DT * rjp[r] * s1) / (g.DH * g.DH);
-                if (type == 4) {
-                    vx[r] += (g.DT * rip[r] * cmem(a.inj.sin_azi)[l] * s0) / (g.DH * g.DH);
-                    vy[r] += (g.DT * rjp[r] * cmem(a.inj.cos_azi)[l] * s0) / (g.DH * g.DH);
-                }
-            } else {
-                if (a.ADJOINT_TYPE == 1) { vx[r] += s0; vy[r] += s1; }
-                if (a.ADJOINT_TYPE == 2) vy[r] += s1;
-                if (a.ADJOINT_TYPE == 3) vx[r] += s0;
-            }
-        }
+        for (int r = 0; r < R; r++)
+            if (live[r])
+                for (int l = first_point(a, a.inj, s, e + r * NX, true); l >= 0; l = gmem(a.inj.next)[l])
+                    inject(a, l, nt, rip[r], rjp[r], vx[r], vy[r]);
     }
 #pragma unroll
     for (int r = 0; r < R; r++)
@@ -438,16 +394,13 @@ __device__ __forceinline__ void str_cell(const StepArgs &a, int s, int blk, int 
     const bool snap_step = (flags & kSnapStep) != 0;
     const bool corr_step = (flags & kCorrStep) != 0;
     const bool rates = snap_step && a.VELOCITY == 1;
-    // bounds of this tile's explosive-source and receiver lists, loaded
-    // before the stencil work so that their latency is hidden behind it
-    int expl = 0, ex0 = 0, ex1 = 0, rc0 = 0, rc1 = 0;
-    if (flags & kForward) {
-        const int so = __builtin_amdgcn_readfirstlane(s * (a.nbx * a.nby + 1) + blk);  // uniform
-        expl = cmem(a.explosive)[s];
-        ex0 = cmem(a.exp.start)[so];
-        ex1 = cmem(a.exp.start)[so + 1];
-        rc0 = cmem(a.rec.start)[so];
-        rc1 = cmem(a.rec.start)[so + 1];
+    // the explosive sources and receivers of this cell, looked up before the
+    // stencil work so that the latency is hidden behind it
+    int ex = -1, rc = -1;
+    if ((flags & kForward) && live) {
+        const int nt_ = a.nbx * a.nby;
+        ex = first_point(a, a.exp, s, e, cmem(a.explosive)[s] && tile_has(a.exp, s, nt_, blk));
+        rc = first_point(a, a.rec, s, e, tile_has(a.rec, s, nt_, blk));
     }
 
     float sxx = 0.0f, syy = 0.0f, sxy = 0.0f, ux = 0.0f, uy = 0.0f, uxy = 0.0f;
@@ -473,16 +426,12 @@ __device__ __forceinline__ void str_cell(const StepArgs &a, int s, int blk, int 
             stress_visc<(L > 0 ? L : 1)>(M.vc, a.eta, a.bip, a.bjm, a.cip, a.cjm, g.DT, vxx, vyx, vxy, vyy, sxx, syy,
                                        sxy, rr, pp, qq, rates, ux, uy, uxy);
         }
-        // explosive sources of this tile, applied after the stress update
+        // explosive sources of this cell, applied after the stress update
         // and before the free surface (src/IFOS2D.c:1758-1773)
-        if (expl) {
-            for (int q = ex0; q < ex1; q++) {
-                const int l = cmem(a.exp.idx)[q];
-                if (cmem(a.exp.ix)[l] != i || cmem(a.exp.iy)[l] != j) continue;
-                const float amp = explosive_amp(a.exp.sig + (long)l * a.NT - 1, nt, a.NT, g.DH);
-                sxx = add_half(sxx, amp);
-                syy = add_half(syy, amp);
-            }
+        for (int l = ex; l >= 0; l = gmem(a.exp.next)[l]) {
+            const float amp = explosive_amp(a.exp.sig + (long)l * a.NT - 1, nt, a.NT, g.DH);
+            sxx = add_half(sxx, amp);
+            syy = add_half(syy, amp);
         }
     }
     if (top) {
@@ -542,13 +491,9 @@ __device__ __forceinline__ void str_cell(const StepArgs &a, int s, int blk, int 
         gmem(a.wc)[wco + e] = w;
         gmem(a.wc_u)[wco + e] = wu;
     }
-    if (flags & kForward) {
-        for (int q = rc0; q < rc1; q++) {
-            const int t = cmem(a.rec.idx)[q];
-            if (cmem(a.rec.ix)[t] != i || cmem(a.rec.iy)[t] != j) continue;
-            gmem(a.seis_vx)[(long)t * a.NT + nt - 1] = vxs[c];
-            gmem(a.seis_vy)[(long)t * a.NT + nt - 1] = vys[c];
-        }
+    for (int t = rc; t >= 0; t = gmem(a.rec.next)[t]) {
+        gmem(a.seis_vx)[(long)t * a.NT + nt - 1] = vxs[c];
+        gmem(a.seis_vy)[(long)t * a.NT + nt - 1] = vys[c];
     }
     if (a.nan_flag && j == g.NY / 2 && i == g.NX / 2) {
         const float v = vys[c];
@@ -718,8 +663,6 @@ __global__ __launch_bounds__(512) void k_fused_step(const StepArgs *__restrict__
         stage(rsxy, &st.sxy[0][0], SY, AX, j0 + 1 - 2 * N, i0 + 1 - 2 * N);
         __syncthreads();
         // ---- velocities of the tile and its rim
-        const int so = __builtin_amdgcn_readfirstlane(s * (a.nbx * a.nby + 1) + blk);  // uniform
-        const int q0 = cmem(a.injx.start)[so], q1 = cmem(a.injx.start)[so + 1];
         for (int q = tid; q < VX * VY; q += kTileX * kTileY) {
             const int ry = q / VX, rx = q - ry * VX;
             const int gj = j0 + 1 - N + ry, gi = i0 + 1 - N + rx;
@@ -761,26 +704,10 @@ __global__ __launch_bounds__(512) void k_fused_step(const StepArgs *__restrict__
                 }
                 vx = vel_new(vx0, g.DT, rip, sxx_x + sxy_y, g.DH);
                 vy = vel_new(vy0, g.DT, rjp, sxy_x + syy_y, g.DH);
-                // point forces / residual injection at this cell, in list order
-                for (int qq = q0; qq < q1; qq++) {
-                    const int l = cmem(a.injx.idx)[qq];
-                    if (cmem(a.injx.ix)[l] != gi || cmem(a.injx.iy)[l] != gj) continue;
-                    const float s0 = cmem(a.injx.sig)[(long)l * a.NT + nt - 1];
-                    const float s1 = cmem(a.injx.sig1)[(long)l * a.NT + nt - 1];
-                    if (a.sw == 0) {
-                        const int type = cmem(a.injx.type)[l];
-                        if (type == 2) vx += (g.DT * rip * s1) / (g.DH * g.DH);
-                        if (type == 3) vy += (g.DT * rjp * s1) / (g.DH * g.DH);
-                        if (type == 4) {
-                            vx += (g.DT * rip * cmem(a.injx.sin_azi)[l] * s0) / (g.DH * g.DH);
-                            vy += (g.DT * rjp * cmem(a.injx.cos_azi)[l] * s0) / (g.DH * g.DH);
-                        }
-                    } else {
-                        if (a.ADJOINT_TYPE == 1) { vx += s0; vy += s1; }
-                        if (a.ADJOINT_TYPE == 2) vy += s1;
-                        if (a.ADJOINT_TYPE == 3) vx += s0;
-                    }
-                }
+                // point forces / residual injection at this cell, in order
+                for (int l = first_point(a, a.inj, s, (long)(gj - 1) * NX + (gi - 1), true); l >= 0;
+                     l = gmem(a.inj.next)[l])
+                    inject(a, l, nt, rip, rjp, vx, vy);
                 if (own) {
                     gmem(wvx)[wo + c] = vx;
                     gmem(wvy)[wo + c] = vy;
@@ -809,13 +736,10 @@ __global__ __launch_bounds__(512) void k_fused_step(const StepArgs *__restrict__
                 W[e] += ((nvx * nvx) + (nvy * nvy));
             }
         }
-        int expl = 0, ex0 = 0, ex1 = 0, rc0 = 0, rc1 = 0;
-        if (fwd) {
-            expl = cmem(a.explosive)[s];
-            ex0 = cmem(a.exp.start)[so];
-            ex1 = cmem(a.exp.start)[so + 1];
-            rc0 = cmem(a.rec.start)[so];
-            rc1 = cmem(a.rec.start)[so + 1];
+        int ex = -1, rc = -1;
+        if (fwd && live) {
+            ex = first_point(a, a.exp, s, e, cmem(a.explosive)[s] && tile_has(a.exp, s, m.ntiles, blk));
+            rc = first_point(a, a.rec, s, e, tile_has(a.rec, s, m.ntiles, blk));
         }
         float sxx = 0.0f, syy = 0.0f, sxy = 0.0f, ux = 0.0f, uy = 0.0f, uxy = 0.0f;
         float rr[L > 0 ? L : 1], pp[L > 0 ? L : 1], qq[L > 0 ? L : 1];
@@ -865,14 +789,10 @@ __global__ __launch_bounds__(512) void k_fused_step(const StepArgs *__restrict__
                 stress_visc<(L > 0 ? L : 1)>(M.vc, a.eta, a.bip, a.bjm, a.cip, a.cjm, g.DT, vxx, vyx, vxy, vyy, sxx,
                                            syy, sxy, rr, pp, qq, rates, ux, uy, uxy);
             }
-            if (expl) {
-                for (int q = ex0; q < ex1; q++) {
-                    const int l = cmem(a.exp.idx)[q];
-                    if (cmem(a.exp.ix)[l] != i || cmem(a.exp.iy)[l] != j) continue;
-                    const float amp = explosive_amp(a.exp.sig + (long)l * a.NT - 1, nt, a.NT, g.DH);
-                    sxx = add_half(sxx, amp);
-                    syy = add_half(syy, amp);
-                }
+            for (int l = ex; l >= 0; l = gmem(a.exp.next)[l]) {
+                const float amp = explosive_amp(a.exp.sig + (long)l * a.NT - 1, nt, a.NT, g.DH);
+                sxx = add_half(sxx, amp);
+                syy = add_half(syy, amp);
             }
         }
         if (top) {
@@ -945,13 +865,9 @@ __global__ __launch_bounds__(512) void k_fused_step(const StepArgs *__restrict__
             gmem(a.wc)[wco + e] = w;
             gmem(a.wc_u)[wco + e] = wu;
         }
-        if (fwd) {
-            for (int q = rc0; q < rc1; q++) {
-                const int t = cmem(a.rec.idx)[q];
-                if (cmem(a.rec.ix)[t] != i || cmem(a.rec.iy)[t] != j) continue;
-                gmem(a.seis_vx)[(long)t * a.NT + nt - 1] = nvx;
-                gmem(a.seis_vy)[(long)t * a.NT + nt - 1] = nvy;
-            }
+        for (int t = rc; t >= 0; t = gmem(a.rec.next)[t]) {
+            gmem(a.seis_vx)[(long)t * a.NT + nt - 1] = nvx;
+            gmem(a.seis_vy)[(long)t * a.NT + nt - 1] = nvy;
         }
         if (a.nan_flag && j == NY / 2 && i == NX / 2) {
             if (isnan(nvy) && *gmem(a.nan_flag) == 0) *gmem(a.nan_flag) = nt;

@@ -123,6 +123,41 @@ __device__ __forceinline__ long mv_index(long c, int k, int L3)
 }
 
 // ---------------------------------------------------------------------------
+// Points at a cell.  first_point: the first one of slot s at interior cell e,
+// -1 when there is none; `any` (uniform): whether the cell's tile has points.
+__device__ __forceinline__ bool tile_has(const PointMap &p, int s, int ntiles, int blk)
+{
+    const int so = __builtin_amdgcn_readfirstlane(s * (ntiles + 1) + blk);  // uniform
+    return cmem(p.start)[so + 1] > cmem(p.start)[so];
+}
+
+__device__ __forceinline__ int first_point(const StepArgs &a, const PointMap &p, int s, long e, bool any)
+{
+    return any ? gmem(p.map)[(long)s * a.plane + e] : -1;
+}
+
+// point force (forward) or residual injection (adjoint) of point l at step nt
+__device__ __forceinline__ void inject(const StepArgs &a, int l, int nt, float rip, float rjp, float &vx, float &vy)
+{
+    const StepGeom &g = a.g;
+    const float s0 = gmem(a.inj.sig)[(long)l * a.NT + nt - 1];
+    const float s1 = gmem(a.inj.sig1)[(long)l * a.NT + nt - 1];
+    if (a.sw == 0) {
+        const int type = gmem(a.inj.type)[l];
+        if (type == 2) vx += (g.DT * rip * s1) / (g.DH * g.DH);
+        if (type == 3) vy += (g.DT * rjp * s1) / (g.DH * g.DH);
+        if (type == 4) {
+            vx += (g.DT * rip * gmem(a.inj.sin_azi)[l] * s0) / (g.DH * g.DH);
+            vy += (g.DT * rjp * gmem(a.inj.cos_azi)[l] * s0) / (g.DH * g.DH);
+        }
+    } else {
+        if (a.ADJOINT_TYPE == 1) { vx += s0; vy += s1; }
+        if (a.ADJOINT_TYPE == 2) vy += s1;
+        if (a.ADJOINT_TYPE == 3) vx += s0;
+    }
+}
+
+// ---------------------------------------------------------------------------
 // 16-bit snapshots.  A tile's values of one field are divided by 2^e, the
 // smallest power of two above their largest magnitude (exact in binary
 // floating point), and rounded to nearest-even BF16 or FP16.
