@@ -231,6 +231,20 @@ class Engine:
         _check(lib().ifos_engine_get_graphs(self.h, C.byref(on)))
         return bool(on.value)
 
+    def set_resident(self, mode):
+        """The whole time loop as one launch: 1 wherever it fits, 0 never, -1 by rule; same bits."""
+        _check(lib().ifos_engine_set_resident(self.h, int(mode)))
+
+    def get_resident(self):
+        """(the next run will take it, the last run did)."""
+        a, b = C.c_int(), C.c_int()
+        _check(lib().ifos_engine_get_resident(self.h, C.byref(a), C.byref(b)))
+        return bool(a.value), bool(b.value)
+
+    def set_resident_wait(self, seconds):
+        """Longest wait for a neighbouring tile before the run is repeated with the per-step kernels."""
+        _check(lib().ifos_engine_set_resident_wait(self.h, C.c_double(seconds)))
+
     def set_launch(self, spb=1, grid=0):
         _check(lib().ifos_engine_set_launch(self.h, spb, grid))
 

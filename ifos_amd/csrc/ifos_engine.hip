@@ -10,6 +10,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -23,6 +24,7 @@
 #include "ifos2d_hip.h"
 #include "ifos2d_opt.h"
 #include "ifos_internal.h"
+#include "ifos_resident.h"
 #include "ifos_step.h"
 
 namespace ifos {
@@ -92,6 +94,12 @@ static hipError_t dfree(void *p)
     std::lock_guard<std::mutex> g(device_lock());
     return hipFree(p);
 }
+
+// longest wait of a workgroup of k_resident for a neighbour, in ticks of the
+// 100 MHz clock: 0.2 s, thousands of time steps.  Past it the workgroups are
+// not all running (another program may hold part of the GPU), the run is given
+// up and repeated with the per-step kernels.
+constexpr unsigned long long kResidentLimit = 20000000ull;
 
 struct ifos_engine {
     ifos_config c;
@@ -200,6 +208,14 @@ struct ifos_engine {
     int gkey[2][6] = {{-1, -1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1, -1}};
     int graph_mode = -1;            // time loop: 1 captured graphs, 0 eager launches, -1 by size (use_graphs)
     int swizzle = 1;
+    // the time loop as one launch (k_resident)
+    int resident_mode = -1;         // 1 wherever it fits, 0 never, -1 by rule (use_resident)
+    bool loop_given = false;        // the caller chose a loop or launch shape of the per-step kernels
+    bool resident_last = false;     // the last run took it
+    int ncu = 0, lds_max = 0;
+    unsigned long long *inbox = nullptr;
+    size_t inbox_words = 0;
+    unsigned long long resident_limit = kResidentLimit;
 };
 
 #define ENG_TRY(expr)       \
@@ -353,6 +369,11 @@ static int engine_create(const ifos_config *cfg, int device, int slots, ifos_eng
     float *b2 = yb + 4 * ys;
     E->psi2_sxx_x = b2; E->psi2_sxy_x = b2 + xs; E->psi2_syy_y = b2 + 2 * xs; E->psi2_sxy_y = b2 + 2 * xs + ys;
 
+    if (hipDeviceGetAttribute(&E->ncu, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess ||
+        hipDeviceGetAttribute(&E->lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, device) != hipSuccess) {
+        ifos_set_error("cannot read the properties of device %d", device);
+        return fail(-1);
+    }
     if (dmalloc(&E->ctl, sizeof(int) * 4) != hipSuccess) return fail(-3);
     hipMemsetAsync(E->ctl, 0, sizeof(int) * 4, E->stream);
     if (dmalloc(&E->explosive, sizeof(int) * slots) != hipSuccess) return fail(-3);
@@ -398,6 +419,7 @@ extern "C" void ifos_engine_destroy(ifos_engine *E)
     dfree(E->tap_m); dfree(E->tap_ij); dfree(E->tap_lohi); dfree(E->tfbuf);
     dfree(E->src_i); dfree(E->src_d); dfree(E->sig); dfree(E->rec_i); dfree(E->seis);
     dfree(E->trace_sums); dfree(E->snap); dfree(E->tiles); dfree(E->point_map);
+    dfree(E->inbox);
     if (E->stream) hipStreamDestroy(E->stream);
     ifos_free_materials(&E->mat);
     delete E;
@@ -692,6 +714,7 @@ static StepArgs step_args(ifos_engine *E, int sw, bool snapshots)
     a.plane = E->plane;
     a.vx = E->vx; a.vy = E->vy; a.sxx = E->sxx; a.syy = E->syy; a.sxy = E->sxy;
     a.vxp1 = E->vxp1; a.vyp1 = E->vyp1;
+    a.ux = E->ux; a.uy = E->uy; a.uxy = E->uxy;
     a.r = E->r; a.p = E->p; a.q = E->q;
     a.ws = E->ws;
     a.ls = E->field;
@@ -861,8 +884,110 @@ static int zero_state(ifos_engine *E)
 {
     HIP_TRY(hipMemsetAsync(E->slab, 0, sizeof(float) * E->ws * E->nslots, E->stream));
     HIP_TRY(hipMemsetAsync(E->psi, 0, sizeof(float) * E->pss * E->nslots, E->stream));
-    HIP_TRY(hipMemsetAsync(E->ctl, 0, sizeof(int) * 2, E->stream));
+    HIP_TRY(hipMemsetAsync(E->ctl, 0, sizeof(int) * 3, E->stream));
     return 0;
+}
+
+// what a run accumulates into, zero before it begins: the state, and the
+// energies of this shot's wavefields (src/IFOS2D.c:1623-1631) or the
+// correlations and the receiver side's energies
+static int zero_run(ifos_engine *E, int sw, bool snapshots)
+{
+    ENG_TRY(zero_state(E));
+    if (sw == 1) HIP_TRY(hipMemsetAsync(E->wcbuf, 0, sizeof(float) * 3 * E->plane * E->nslots, E->stream));
+    if (!E->ep_mode || (sw == 0 && !snapshots)) return 0;
+    for (int k = 0; k < E->nslots; k++) {
+        const long o = 2 * k * E->plane + (sw == 0 ? 0 : E->plane), n = (sw == 0 ? 2 : 1) * E->plane;
+        HIP_TRY(hipMemsetAsync(E->wbuf + o, 0, sizeof(float) * n, E->stream));
+        if (E->ep_fp64) HIP_TRY(hipMemsetAsync(E->wbuf64 + o, 0, sizeof(double) * n, E->stream));
+    }
+    return 0;
+}
+
+// ---------------------------------------------------------------------------
+// the time loop as one launch
+// ---------------------------------------------------------------------------
+static ResidentPlan plan_of(const ifos_engine *E, int nslots)
+{
+    return resident_plan(geom(E), E->c.L, nslots, E->snap_prec, E->ncu, (size_t)E->lds_max);
+}
+
+// Taken wherever the shots' tiles fit the chip one per compute unit, unless
+// the caller chose a loop or launch shape of the per-step kernels.
+static bool use_resident(const ifos_engine *E)
+{
+    if (E->resident_mode == 0) return false;
+    if (E->resident_mode < 0 && (E->graph_mode >= 0 || E->loop_given || E->fused)) return false;
+    return E->nslots > 0 && plan_of(E, E->nslots).rows > 0;
+}
+
+// One resident run at a time on a device: two that share the compute units
+// could each hold what the other waits for until both give up.  A run that
+// finds the device taken uses the per-step kernels.
+struct ResidentTurn {
+    static constexpr int kDevices = 64;
+    static std::atomic<bool> &taken(int device)
+    {
+        static std::atomic<bool> t[kDevices];
+        return t[device];
+    }
+    int device;
+    bool mine;
+    explicit ResidentTurn(int d) : device(d), mine(d >= 0 && d < kDevices && !taken(d).exchange(true)) {}
+    ~ResidentTurn()
+    {
+        if (mine) taken(device) = false;
+    }
+};
+
+// done: the run is complete; false: it was not taken, or given up (zero_run
+// must precede another attempt)
+static int run_resident(ifos_engine *E, int sw, bool snapshots, bool &done)
+{
+    done = false;
+    const ResidentPlan p = plan_of(E, E->nslots);
+    const size_t need = (size_t)p.nwg * 2 * p.words;
+    if (need > E->inbox_words) {
+        dfree(E->inbox);
+        E->inbox = nullptr;
+        E->inbox_words = 0;
+        HIP_TRY(dmalloc(&E->inbox, sizeof(unsigned long long) * need));
+        E->inbox_words = need;
+    }
+    StepArgs a = step_args(E, sw, snapshots);
+    a.base = nullptr;
+    const StepArgs *da = nullptr;
+    ENG_TRY(upload_args(E, a, 3, &da));
+    HIP_TRY(hipMemsetAsync(E->inbox, 0, sizeof(unsigned long long) * need, E->stream));
+    ResidentArgs r;
+    memset(&r, 0, sizeof r);
+    r.a = da;
+    r.inbox = E->inbox;
+    r.stop = E->ctl + 2;
+    r.limit = E->resident_limit;
+    HIP_TRY(launch_resident(a, r, p, E->stream));
+    int stop = 0;
+    HIP_TRY(hipMemcpyAsync(&stop, E->ctl + 2, sizeof stop, hipMemcpyDeviceToHost, E->stream));
+    HIP_TRY(hipStreamSynchronize(E->stream));
+    done = stop == 0;
+    if (done) E->last_set = 0;
+    return 0;
+}
+
+// a forward (sw 0) or adjoint run of NT steps from a zero state
+static int run_steps(ifos_engine *E, int sw, bool snapshots)
+{
+    ENG_TRY(zero_run(E, sw, snapshots));
+    E->resident_last = false;
+    if (use_resident(E)) {
+        ResidentTurn turn(E->device);
+        if (turn.mine) {
+            ENG_TRY(run_resident(E, sw, snapshots, E->resident_last));
+            if (E->resident_last) return 0;
+            ENG_TRY(zero_run(E, sw, snapshots));
+        }
+    }
+    return run_loop(E, sw, snapshots);
 }
 
 static size_t snapshot_bytes(const ifos_config &c, int prec)
@@ -908,13 +1033,7 @@ extern "C" int ifos_engine_forward(ifos_engine *E, int store_snapshots)
     if (store_snapshots) ENG_TRY(ensure_snapshots(E));
     E->snap_valid = false;
     E->slot_grad_valid = false;
-    ENG_TRY(zero_state(E));
-    // energies of this shot's wavefields start at zero (src/IFOS2D.c:1623-1631)
-    if (E->ep_mode && store_snapshots)
-        HIP_TRY(hipMemsetAsync(E->wbuf, 0, sizeof(float) * 2 * E->plane * E->nslots, E->stream));
-    if (E->ep_mode && store_snapshots && E->ep_fp64)
-        HIP_TRY(hipMemsetAsync(E->wbuf64, 0, sizeof(double) * 2 * E->plane * E->nslots, E->stream));
-    ENG_TRY(run_loop(E, 0, store_snapshots != 0));
+    ENG_TRY(run_steps(E, 0, store_snapshots != 0));
     ENG_TRY(check_nan(E));
     E->snap_valid = store_snapshots != 0;
     return 0;
@@ -1353,9 +1472,7 @@ extern "C" int ifos_engine_adjoint(ifos_engine *E)
         return ifos_set_error("adjoint needs a forward run with snapshots on the current model and shot"), -2;
     if (!E->tiles || !E->model_set) return ifos_set_error("adjoint needs set_model and set_shot"), -2;
     E->slot_grad_valid = false;
-    ENG_TRY(zero_state(E));
-    HIP_TRY(hipMemsetAsync(E->wcbuf, 0, sizeof(float) * 3 * E->plane * E->nslots, E->stream));
-    ENG_TRY(run_loop(E, 1, false));
+    ENG_TRY(run_steps(E, 1, false));
     GradArgs ga;
     memset(&ga, 0, sizeof ga);
     if (E->ep_mode) ENG_TRY(energy_weights(E, ga));
@@ -1420,6 +1537,7 @@ extern "C" int ifos_engine_set_fused(ifos_engine *E, int on)
         return ifos_set_error("the one-kernel step has no periodic sides (BOUNDARY 1): its tiles form their "
                               "neighbours' velocities from stresses beyond the halo copies"), -2;
     HIP_TRY(hipStreamSynchronize(E->stream));
+    E->loop_given = true;
     if ((on != 0) != E->fused) drop_graphs(E);
     E->fused = on != 0;
     return 0;
@@ -1474,6 +1592,16 @@ extern "C" size_t ifos_engine_bytes(const ifos_config *c, int slots, int snap_pr
     b += (sizeof(float) * c->NT + 3 * sizeof(int) + 2 * sizeof(double)) * (size_t)nsrc_total;
     b += (3 * sizeof(int) + 2 * sizeof(double)) * (size_t)ntr_total;
     if (snapshots) b += snapshot_bytes(*c, snap_prec) * slots + 256;
+    // inboxes of the one-launch time loop, at most one workgroup of the
+    // tallest tile on each of 256 compute units
+    StepGeom g{};
+    g.NX = c->NX; g.NY = c->NY; g.N = N; g.FREE_SURF = c->FREE_SURF; g.BOUNDARY = c->BOUNDARY;
+    size_t inbox = 0;
+    for (int s = 1; s <= std::min(slots, 256); s++) {
+        const ResidentPlan p = resident_plan(g, c->L, s, snap_prec, 256, 163840);
+        if (p.rows) inbox = std::max(inbox, sizeof(unsigned long long) * 2 * (size_t)p.nwg * p.words);
+    }
+    b += inbox;
     return b;
 }
 
@@ -1515,6 +1643,7 @@ extern "C" int ifos_engine_set_launch(ifos_engine *E, int spb, int grid)
 {
     if (spb != 1 && spb != 2 && spb != 4) return ifos_set_error("shots per workgroup must be 1, 2 or 4"), -2;
     if (grid < 0 || grid % 8) return ifos_set_error("persistent grid must be 0 or a positive multiple of 8"), -2;
+    E->loop_given = true;
     E->shape.spb = spb;
     E->shape.grid = grid;
     E->shape.grid_v = grid;
@@ -1541,6 +1670,26 @@ extern "C" int ifos_engine_get_graphs(ifos_engine *E, int *on)
     return 0;
 }
 
+extern "C" int ifos_engine_set_resident(ifos_engine *E, int mode)
+{
+    if (mode < -1 || mode > 1) return ifos_set_error("resident mode must be -1, 0 or 1"), -2;
+    E->resident_mode = mode;
+    return 0;
+}
+
+extern "C" int ifos_engine_get_resident(ifos_engine *E, int *next, int *last)
+{
+    if (next) *next = use_resident(E) ? 1 : 0;
+    if (last) *last = E->resident_last ? 1 : 0;
+    return 0;
+}
+
+extern "C" int ifos_engine_set_resident_wait(ifos_engine *E, double seconds)
+{
+    E->resident_limit = seconds < 0 ? kResidentLimit : (unsigned long long)(std::min(seconds, 10.0) * 1e8);
+    return 0;
+}
+
 extern "C" int ifos_engine_get_launch(ifos_engine *E, int *spb, int *grid)
 {
     *spb = E->shape.spb;
@@ -1551,6 +1700,7 @@ extern "C" int ifos_engine_get_launch(ifos_engine *E, int *spb, int *grid)
 extern "C" int ifos_engine_set_velocity_rows(ifos_engine *E, int rows)
 {
     if (rows != 1 && rows != 2 && rows != 4) return ifos_set_error("velocity rows per thread must be 1, 2 or 4"), -2;
+    E->loop_given = true;
     E->shape.rows_v = rows;
     if (rows != 2) E->shape.lds_v = 0;
     return 0;
@@ -1564,6 +1714,7 @@ extern "C" int ifos_engine_get_velocity_rows(ifos_engine *E, int *rows)
 
 extern "C" int ifos_engine_set_velocity_lds(ifos_engine *E, int on)
 {
+    E->loop_given = true;
     E->shape.lds_v = on ? 1 : 0;
     if (on) E->shape.rows_v = 2;
     return 0;
@@ -1577,6 +1728,7 @@ extern "C" int ifos_engine_get_velocity_lds(ifos_engine *E, int *on)
 
 extern "C" int ifos_engine_set_work_order(ifos_engine *E, int slot_major)
 {
+    E->loop_given = true;
     E->shape.order = slot_major ? 1 : 0;
     return 0;
 }

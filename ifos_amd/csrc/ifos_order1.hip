@@ -1,4 +1,5 @@
 // ifos_order1.hip -- time-loop kernels of FDORDER 2.
+#include "ifos_resident_kernels.h"
 #include "ifos_step_kernels.h"
 
 namespace ifos {
@@ -6,5 +7,7 @@ namespace ifos {
 template void vel_n<1>(const StepArgs &a, const StepArgs *da, const LaunchShape &ls, int k, hipStream_t s);
 template void str_n<1>(const StepArgs &a, const StepArgs *da, const LaunchShape &ls, int k, hipStream_t s);
 template void fused_n<1>(const StepArgs &a, const StepArgs *da, const LaunchShape &ls, int k, hipStream_t s);
+template size_t resident_lds<1>(int th);
+template hipError_t resident_n<1>(int L, const ResidentArgs &r, const ResidentPlan &p, hipStream_t s);
 
 }  // namespace ifos

@@ -39,6 +39,8 @@ struct StepArgs {
     // per-slot padded grids (stride ws floats between slots)
     float *vx, *vy, *sxx, *syy, *sxy;
     float *vxp1, *vyp1;        // adjoint only
+    float *ux, *uy, *uxy;      // k_resident, forward: values of a 16-bit snapshot until their scale is known
+                               // (vxp1, vyp1 likewise)
     float *r, *p, *q;
     long ws;
     long ls;                   // plane stride of the memory variables

@@ -4,6 +4,7 @@
 #include <algorithm>
 #include <vector>
 
+#include "ifos_resident.h"
 #include "ifos_step.h"
 
 namespace ifos {
@@ -14,6 +15,10 @@ template <int N>
 void str_n(const StepArgs &a, const StepArgs *da, const LaunchShape &ls, int k, hipStream_t s);
 template <int N>
 void fused_n(const StepArgs &a, const StepArgs *da, const LaunchShape &ls, int k, hipStream_t s);
+template <int N>
+size_t resident_lds(int th);
+template <int N>
+hipError_t resident_n(int L, const ResidentArgs &r, const ResidentPlan &p, hipStream_t s);
 
 __global__ void k_tick(int *base, int by)
 {
@@ -108,6 +113,67 @@ void launch_fused_step(const StepArgs &a, const StepArgs *da, const LaunchShape 
     case 5: fused_n<5>(a, da, ls, k, s); break;
     case 6: fused_n<6>(a, da, ls, k, s); break;
     default: break;
+    }
+}
+
+static size_t lds_of(int N, int th)
+{
+    switch (N) {
+    case 1: return resident_lds<1>(th);
+    case 2: return resident_lds<2>(th);
+    case 3: return resident_lds<3>(th);
+    case 4: return resident_lds<4>(th);
+    case 5: return resident_lds<5>(th);
+    default: return resident_lds<6>(th);
+    }
+}
+
+// One workgroup per compute unit at most, all of them resident at once.  The
+// tile is as low as that allows (the steps of a small grid cost latency, not
+// throughput: more workgroups, less work in each), at least as high as the
+// stencil reaches, and on the free surface as the rows mirrored above it.
+ResidentPlan resident_plan(const StepGeom &g, int L, int nslots, int snap_prec, int ncu, size_t lds_max)
+{
+    ResidentPlan p;
+    const int most = resident_max_rows(L), nbx = (g.NX + kTileX - 1) / kTileX;
+    // periodic sides wrap the halo, which may span two tiles there
+    if (g.BOUNDARY || most == 0 || nslots < 1 || (long)nbx * nslots > ncu) return p;
+    const int across = ncu / (nbx * nslots);  // tile rows per slot that fit
+    int th = std::max((g.NY + across - 1) / across, g.N + (g.FREE_SURF ? 1 : 0));
+    for (int rows = 1; rows <= most; rows++) {
+        int ty = (th + rows - 1) / rows;
+        // the scales of 16-bit snapshots belong to 64x8 tiles
+        while (snap_prec && ty * rows % kTileY) ty++;
+        if (ty > kResidentThreads / kTileX) continue;
+        p.ty = ty;
+        p.th = ty * rows;
+        p.tiles_y = (g.NY + p.th - 1) / p.th;
+        p.nwg = nbx * p.tiles_y * nslots;
+        p.words = (2 * g.N - 1) * 2 * (kTileX + p.th);
+        p.lds = lds_of(g.N, p.th);
+        if (p.lds + 64 <= lds_max) p.rows = rows;
+        return p;
+    }
+    return p;
+}
+
+hipError_t launch_resident(const StepArgs &a, ResidentArgs r, const ResidentPlan &p, hipStream_t s)
+{
+    r.words = p.words;
+    r.th = p.th;
+    r.ty = p.ty;
+    r.tiles_y = p.tiles_y;
+    r.ntile = a.nbx * p.tiles_y;
+    r.nwg = p.nwg;
+    r.per = (p.nwg + 7) / 8;
+    switch (a.g.N) {
+    case 1: return resident_n<1>(a.L, r, p, s);
+    case 2: return resident_n<2>(a.L, r, p, s);
+    case 3: return resident_n<3>(a.L, r, p, s);
+    case 4: return resident_n<4>(a.L, r, p, s);
+    case 5: return resident_n<5>(a.L, r, p, s);
+    case 6: return resident_n<6>(a.L, r, p, s);
+    default: return hipErrorInvalidValue;
     }
 }
 

@@ -137,9 +137,11 @@ __device__ __forceinline__ int first_point(const StepArgs &a, const PointMap &p,
 }
 
 // point force (forward) or residual injection (adjoint) of point l at step nt
-__device__ __forceinline__ void inject(const StepArgs &a, int l, int nt, float rip, float rjp, float &vx, float &vy)
+// (A: the argument block through a plain or a constant-space reference)
+template <class A>
+__device__ __forceinline__ void inject(A &a, int l, int nt, float rip, float rjp, float &vx, float &vy)
 {
-    const StepGeom &g = a.g;
+    const auto &g = a.g;
     const float s0 = gmem(a.inj.sig)[(long)l * a.NT + nt - 1];
     const float s1 = gmem(a.inj.sig1)[(long)l * a.NT + nt - 1];
     if (a.sw == 0) {
@@ -161,7 +163,8 @@ __device__ __forceinline__ void inject(const StepArgs &a, int l, int nt, float r
 // 16-bit snapshots.  A tile's values of one field are divided by 2^e, the
 // smallest power of two above their largest magnitude (exact in binary
 // floating point), and rounded to nearest-even BF16 or FP16.
-__device__ __forceinline__ bool has_snap(const StepArgs &a) { return a.snap[0] || a.snap16[0]; }
+template <class A>
+__device__ __forceinline__ bool has_snap(A &a) { return a.snap[0] || a.snap16[0]; }
 
 __device__ __forceinline__ int scale_exp(float m)
 {

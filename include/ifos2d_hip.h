@@ -128,6 +128,19 @@ int  ifos_engine_shot_misfit(ifos_engine *e, double *per_shot);
  * what the next run will use. */
 int  ifos_engine_set_graphs(ifos_engine *e, int mode);
 int  ifos_engine_get_graphs(ifos_engine *e, int *on);
+/* The whole time loop as one launch: each compute unit keeps a tile of the
+ * grid for the run and exchanges edge lines with its neighbours' after every
+ * half step.  mode 1 takes it wherever the shots' tiles fit the chip, 0
+ * never, -1 (the default) wherever they fit unless the caller chose a loop or
+ * a launch shape of the per-step kernels (set_graphs, set_launch,
+ * set_work_order, set_velocity_rows, set_velocity_lds, set_fused).  Same bits
+ * either way.  A workgroup that waits longer than set_resident_wait's seconds
+ * (default 0.2, negative restores it) gives the run up, and it is repeated
+ * with the per-step kernels.  get_resident reports whether the next run will
+ * take it, and whether the last one did. */
+int  ifos_engine_set_resident(ifos_engine *e, int mode);
+int  ifos_engine_get_resident(ifos_engine *e, int *next, int *last);
+int  ifos_engine_set_resident_wait(ifos_engine *e, double seconds);
 int  ifos_engine_set_launch(ifos_engine *e, int spb, int grid);
 int  ifos_engine_get_launch(ifos_engine *e, int *spb, int *grid);
 /* The persistent grids of the velocity and the stress step (set_launch sets
