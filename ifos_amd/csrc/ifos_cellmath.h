@@ -195,14 +195,44 @@ __device__ __forceinline__ float vel_new(float v, float DT, float r, float s, fl
 // acceleration kept for the density correlation (sw == 0)
 __device__ __forceinline__ float vel_rate(float r, float s, float DH) { return r * s / DH; }
 
+// x / d, correctly rounded, from r = 1.0 / (double)d: one conversion, one
+// FP64 product and one rounding instead of the eleven-instruction division
+// (the velocity step divides twice a cell by DH, an absorbing cell twice a
+// half step and strip by K).  The product is within 2^-52 of the quotient; a
+// quotient of two 24-bit significands that is not a float is at least 2^-49
+// (relative) from the middle of two floats, and never in the middle, so
+// rounding the product rounds the quotient.  Only a subnormal quotient can be
+// a tie; those divide.  Infinities, NaN and signed zeros pass through.
+__device__ __forceinline__ float div_by(float x, float d, double r)
+{
+    const float q = (float)((double)x * r);
+    if (__builtin_expect(__builtin_amdgcn_classf(q, 0x90), 0)) return x / d;  // -subnormal, +subnormal
+    return q;
+}
+
+// two quotients with one look for subnormal ones
+__device__ __forceinline__ void div_by2(float &x, float &y, float dx, float dy, double rx, double ry)
+{
+    const float qx = (float)((double)x * rx), qy = (float)((double)y * ry);
+    if (__builtin_expect(__builtin_amdgcn_classf(qx, 0x90) | __builtin_amdgcn_classf(qy, 0x90), 0)) {
+        x = x / dx;
+        y = y / dy;
+        return;
+    }
+    x = qx;
+    y = qy;
+}
+
 // elastic stress update (src/update_s_elastic_PML.c:232-234): returns the
-// new sxx, syy, sxy
-__device__ __forceinline__ void stress_elastic(float f, float gl, float fipjp, float vxx, float vyx, float vxy,
+// new sxx, syy, sxy; f2 is 2 f (exact).  The FP64 products of two floats are
+// exact, so fusing them into the sums that follow changes no bit.
+__device__ __forceinline__ void stress_elastic(float f2, float gl, float fipjp, float vxx, float vyx, float vxy,
                                                float vyy, float &sxx, float &syy, float &sxy)
 {
     sxy = sxy + fipjp * (vyx + vxy);
-    sxx = (float)((double)sxx + ((double)(gl * (vxx + vyy)) + (2.0 * (double)f * (double)vxx)));
-    syy = (float)((double)syy + ((double)(gl * (vxx + vyy)) + (2.0 * (double)f * (double)vyy)));
+    const double gd = (double)(gl * (vxx + vyy)), df = (double)f2;
+    sxx = (float)((double)sxx + __builtin_fma(df, (double)vxx, gd));
+    syy = (float)((double)syy + __builtin_fma(df, (double)vyy, gd));
 }
 
 // elastic stress rates (src/update_s_elastic_PML.c:236-238)
@@ -237,17 +267,41 @@ __device__ __forceinline__ void visc_coeffs(int L, float DT, float mu, float pi,
     c.g = (float)((double)(pi * DT) * (1.0 + (double)(L * taup)));
 }
 
+// what the stress update reads of a cell's coefficients: 2 f, g, fipjp, and
+// per mechanism 2 d, e, dip, formed as (modulus*eta_l)*tau like
+// src/prepare_update_s.c:75-77 (the doublings are exact)
+template <int L>
+struct ViscUpdate {
+    float f2, g, fipjp;
+    float d2[L], e[L], dip[L];
+};
+
+template <int L>
+__device__ __forceinline__ void visc_update(const ViscCell &c, const float *eta, ViscUpdate<L> &u)
+{
+    u.f2 = 2.0f * c.f;
+    u.g = c.g;
+    u.fipjp = c.fipjp;
+#pragma unroll
+    for (int l = 0; l < L; l++) {
+        u.dip[l] = c.muipjp * eta[l + 1] * c.tausipjp;
+        u.d2[l] = 2.0f * (c.mu * eta[l + 1] * c.taus);
+        u.e[l] = c.pi * eta[l + 1] * c.taup;
+    }
+}
+
 // viscoelastic stress update with L memory variables
 // (src/update_s_visc_PML.c:486-514).  r/p/q hold the old memory variables on
-// entry and the new ones on exit.  d/e/dip per mechanism are formed as
-// (modulus*eta_l)*tau like src/prepare_update_s.c:75-77.
+// entry and the new ones on exit.  FP64 products of two floats are exact, so
+// fusing them into the sums that follow changes no bit.  DT serves the rates
+// only; the rest takes DT / 2.
 template <int L>
-__device__ __forceinline__ void stress_visc(const ViscCell &c, const float *eta, const float *bip, const float *bjm,
-                                            const float *cip, const float *cjm, float DT, float vxx, float vyx,
+__device__ __forceinline__ void stress_visc(const ViscUpdate<L> &c, const float *bip, const float *bjm,
+                                            const float *cip, const float *cjm, float dthalbe, float DT, float vxx,
+                                            float vyx,
                                             float vxy, float vyy, float &sxx, float &syy, float &sxy, float *r,
                                             float *p, float *q, bool rates, float &ux, float &uy, float &uxy)
 {
-    const float dthalbe = DT / 2.0;
     float sumr = 0.0f, sump = 0.0f, sumq = 0.0f;
 #pragma unroll
     for (int l = 0; l < L; l++) {
@@ -255,28 +309,26 @@ __device__ __forceinline__ void stress_visc(const ViscCell &c, const float *eta,
         sump += p[l];
         sumq += q[l];
     }
+    const double dx = (double)vxx, dy = (double)vyy, f2 = (double)c.f2;
+    const double gd = (double)(c.g * (vxx + vyy));
     sxy = sxy + ((c.fipjp * (vxy + vyx)) + (dthalbe * sumr));
-    sxx = (float)((double)sxx + (((double)(c.g * (vxx + vyy)) - (2.0 * (double)c.f * (double)vyy)) +
-                                 (double)(dthalbe * sump)));
-    syy = (float)((double)syy + (((double)(c.g * (vxx + vyy)) - (2.0 * (double)c.f * (double)vxx)) +
-                                 (double)(dthalbe * sumq)));
+    sxx = (float)((double)sxx + (__builtin_fma(-f2, dy, gd) + (double)(dthalbe * sump)));
+    syy = (float)((double)syy + (__builtin_fma(-f2, dx, gd) + (double)(dthalbe * sumq)));
     if (rates) {
-        const double f2 = (2.0 * (double)c.f) / (double)DT;
+        const double fr = f2 / (double)DT, gr = (double)((c.g / DT) * (vxx + vyy));
         uxy = (float)((double)((c.fipjp / DT) * (vxy + vyx)) + (0.5 * (double)sumr));
-        ux = (float)(((double)((c.g / DT) * (vxx + vyy)) - (f2 * (double)vyy)) + (0.5 * (double)sump));
-        uy = (float)(((double)((c.g / DT) * (vxx + vyy)) - (f2 * (double)vxx)) + (0.5 * (double)sumq));
+        ux = (float)((gr - (fr * dy)) + (0.5 * (double)sump));
+        uy = (float)((gr - (fr * dx)) + (0.5 * (double)sumq));
     }
     sumr = sump = sumq = 0.0f;
 #pragma unroll
     for (int l = 0; l < L; l++) {
-        const float dip = c.muipjp * eta[l + 1] * c.tausipjp;
-        const float d = c.mu * eta[l + 1] * c.taus;
-        const float e = c.pi * eta[l + 1] * c.taup;
-        r[l] = bip[l + 1] * (r[l] * cip[l + 1] - (dip * (vxy + vyx)));
+        const double d2 = (double)c.d2[l];
+        r[l] = bip[l + 1] * (r[l] * cip[l + 1] - (c.dip[l] * (vxy + vyx)));
         p[l] = (float)((double)bjm[l + 1] *
-                       ((double)(p[l] * cjm[l + 1] - (e * (vxx + vyy))) + (2.0 * (double)d * (double)vyy)));
+                       __builtin_fma(d2, dy, (double)(p[l] * cjm[l + 1] - (c.e[l] * (vxx + vyy)))));
         q[l] = (float)((double)bjm[l + 1] *
-                       ((double)(q[l] * cjm[l + 1] - (e * (vxx + vyy))) + (2.0 * (double)d * (double)vxx)));
+                       __builtin_fma(d2, dx, (double)(q[l] * cjm[l + 1] - (c.e[l] * (vxx + vyy)))));
         sumr += r[l];
         sump += p[l];
         sumq += q[l];

@@ -7,13 +7,16 @@
 // workgroup hands the N edge lines its neighbours read to their inboxes in
 // device memory and waits for theirs; nothing else synchronises the tiles.
 //
-// What bounds it: on small grids the latency of the two exchanges per step
-// (about 2 us each: a write-through store, then the neighbour's polling load),
-// on larger ones the arithmetic of the tile.  The per-step kernels pay two
-// launches a step, each with its ramp, drain and cold loads.  Time per step,
-// per-step kernels and this, FDORDER 8, L=2 (us): 1024x128 11.0 / 6.8,
-// 1024x256 13.2 / 8.1, 1024x512 20.0 / 13.8; elastic FDORDER 4: 1024x128
-// 9.4 / 5.5, 1024x768 17.5 / 11.4.
+// What bounds it: with one row of cells per thread the latency of a half step,
+// a chain of instructions more than of memory (400x200 elastic, FDORDER 4,
+// 3.7 us a step: 1.7 update, 0.7 polling and unpacking, 0.8 sending, 0.3 waiting
+// for the write-through stores that the polling loads queue behind, 0.2 for
+// neighbours), so the loop keeps divisions, address arithmetic and anything rare
+// out of its registers and its path; with more rows the instructions issued.
+// The per-step kernels pay two launches a step, each with its ramp, drain and
+// cold loads.  Time per forward step, those and this (us): FDORDER 8, L=2:
+// 1024x256 13.2 / 5.6, 1024x512 20.0 / 13.0, 1024x768 26.5 / 21.4; elastic:
+// 1200x600 FDORDER 8 18.9 / 11.4, 1024x256 FDORDER 4 10.2 / 5.1.
 #pragma once
 #include "ifos_step.h"
 
@@ -23,11 +26,13 @@ constexpr int kResidentThreads = 1024;  // largest workgroup: 64 columns x 16 ro
 
 // Rows of cells per thread the kernel is compiled for, by the number of
 // relaxation mechanisms (0: not compiled).  1024 threads share a compute unit's
-// registers, 128 each; beyond these counts so much of a tile spills to scratch
-// that the per-step kernels win: 1700x350, L=2, FDORDER 8 (three rows) took
-// 77 ms a shot gradient of 1500 steps against their 75 ms, 1024x1024 elastic
-// (four rows) 23.4 us a step against 24.4 and no gain over a gradient.
-constexpr int resident_max_rows(int L) { return L == 0 ? 3 : L <= 3 ? 2 : 0; }
+// registers, 128 each; with these counts at most a few dozen values spill and
+// the run is faster than the per-step kernels' (us per forward step of a full
+// chip, FDORDER 8: elastic, four rows 25.1 / 17.3, L=2, three rows 26.5 / 21.4,
+// L=3, two rows 22.0 / 16.4).
+constexpr int resident_max_rows(int L) { return L == 0 ? 4 : L <= 2 ? 3 : L <= 3 ? 2 : 0; }
+
+constexpr int kWordsPerThread = 3;  // inbox words a thread polls, one row per thread
 
 // A line of the inbox is one word per cell: the value in the low half, the
 // step it belongs to in the high half, written and read as one 64-bit atomic,

@@ -21,7 +21,12 @@ struct ResLds {
     __host__ __device__ static int sxx(int th) { return 3 * (th + 2 * N) * W; }
     __host__ __device__ static int syy(int th) { return 3 * (th + 2 * N) * W + th * W; }
     __host__ __device__ static int maxima(int th) { return syy(th) + (th + 2 * N) * kTileX; }
-    __host__ __device__ static int total(int th) { return maxima(th) + 5 * th; }
+    // CPML profiles of the columns (6 floats, then 2 doubles, [.][64]) and of
+    // the rows ([row] of 6 floats and 2 doubles), moduli of the surface row
+    __host__ __device__ static int xprof(int th) { return (maxima(th) + 5 * th + 1) / 2 * 2; }
+    __host__ __device__ static int yprof(int th) { return xprof(th) + 10 * kTileX; }
+    __host__ __device__ static int surface(int th) { return yprof(th) + 10 * th; }
+    __host__ __device__ static int total(int th) { return surface(th) + 4 * kTileX; }
 };
 
 // The argument block, read afresh: what a block of code needs of it is loaded
@@ -34,6 +39,16 @@ __device__ __forceinline__ ArgPtr afresh(ArgPtr p)
     return p;
 }
 __device__ __forceinline__ unsigned afresh(unsigned v)
+{
+    asm volatile("" : "+v"(v));
+    return v;
+}
+__device__ __forceinline__ int afresh_uniform(int v)
+{
+    asm volatile("" : "+s"(v));
+    return v;
+}
+__device__ __forceinline__ float afresh(float v)
 {
     asm volatile("" : "+v"(v));
     return v;
@@ -67,8 +82,8 @@ __device__ __forceinline__ void send_word(unsigned long long *box, unsigned word
 }
 
 template <int N>
-__device__ __forceinline__ void send_y(const ResidentArgs &ra, int sides, unsigned up, unsigned dn, int r, int tx, float p,
-                                       float q, int tag)
+__device__ __forceinline__ void send_y(const ResidentArgs &ra, int sides, unsigned up, unsigned dn, int r, int tx,
+                                       float p, float q, int tag)
 {
     // up: word 0 of the "from below" lines of the tile above; dn: word 0 of
     // the "from above" lines of the tile below; r is uniform in a wavefront
@@ -84,72 +99,100 @@ __device__ __forceinline__ void send_y(const ResidentArgs &ra, int sides, unsign
 }
 
 template <int N>
-__device__ __forceinline__ void send_x(const ResidentArgs &ra, const XDest &d, int r, float p, float q, int tag)
+__device__ __forceinline__ void send_x(const ResidentArgs &ra, const XDest &d, unsigned half, int r, float p, float q,
+                                       int tag)
 {
-    if (d.p >= 0) send_word(ra.inbox, afresh(d.p) + r * (2 * N - 1), p, tag);
-    if (d.q >= 0) send_word(ra.inbox, afresh(d.q) + r * (2 * N - 1), q, tag);
+    if (d.p >= 0) send_word(ra.inbox, afresh((unsigned)d.p) + half + r * (2 * N - 1), p, tag);
+    if (d.q >= 0) send_word(ra.inbox, afresh((unsigned)d.q) + half + r * (2 * N - 1), q, tag);
 }
 
-// Take this half step's halo out of the inbox `in` into LDS: py and qy are
-// the fields read from below and above, px and qx those from the sides, each
-// given by the LDS offset of its row 0, column 0.  Every thread polls its own
-// words.  false: a neighbour did not answer within ra.limit, or another
-// workgroup gave up.
+// Where inbox word q of a tile goes, as the LDS offset of its cell for the
+// half step whose fields are given by their offsets of row 0, column 0 and
+// row strides (py, qy from below and above, px, qx from the sides); side: the
+// neighbour it comes from.
 template <int N>
-__device__ __forceinline__ bool receive(const ResidentArgs &ra, const unsigned long long *in_, int sides, int tag,
-                                        float *lds, int py, int spy, int qy, int sqy, int px, int spx, int qx, int sqx)
+__device__ __forceinline__ int word_cell(int q, int th, int py, int spy, int qy, int sqy, int px, int spx, int qx,
+                                         int sqx, int &side)
 {
-    constexpr int M = 2 * N - 1, U = 2;
+    constexpr int M = 2 * N - 1;
+    if (q < 2 * M * kTileX) {
+        const bool above = q >= M * kTileX;
+        const int k = above ? q - M * kTileX : q, l = k / kTileX, x = k % kTileX;
+        side = above ? kAbove : kBelow;
+        if (!above) return l < N ? py + (th + l) * spy + x : qy + (th + l - N) * sqy + x;
+        return l < N - 1 ? py + (l - (N - 1)) * spy + x : qy + (l - (N - 1) - N) * sqy + x;
+    }
+    const int h = q - 2 * M * kTileX;
+    const bool left = h >= M * th;
+    const int k = left ? h - M * th : h, r = k / M, l = k % M;
+    side = left ? kLeft : kRight;
+    if (!left) return l < N ? px + r * spx + kTileX + l : qx + r * sqx + kTileX + l - N;
+    return l < N - 1 ? px + r * spx + l - (N - 1) : qx + r * sqx + l - (N - 1) - N;
+}
+
+// inbox words per thread: resident_plan keeps one-row tiles high enough for
+// three; of the others the lowest have the most (16 rows of R - 1 cells did not
+// hold them)
+template <int N, int R>
+constexpr int words_per_thread()
+{
+    const int ty = 16 * (R - 1) / R + 1;
+    return R == 1 ? kWordsPerThread : ((2 * N - 1) * 2 * (kTileX + R * ty) + kTileX * ty - 1) / (kTileX * ty);
+}
+
+// CPML profile values of a column or row, with the reciprocals for div_by
+struct Profile {
+    float K, a, b, Kh, ah, bh;
+    double rK, rKh;
+};
+
+// two derivatives through an absorbing strip: new memory values m and n, then
+// d / K + m.  (Where every K is 1 the division returns d.)
+__device__ __forceinline__ void absorb(float &d, float &m, float Kd, double rd, float ad, float bd, float &f, float &n,
+                                       float Kf, double rf, float af, float bf)
+{
+    m = bd * m + ad * d;
+    n = bf * n + af * f;
+    div_by2(d, f, Kd, Kf, rd, rf);
+    d = d + m;
+    f = f + n;
+}
+
+// Take a half step's halo out of the inbox into LDS.  Thread t polls words t,
+// t + threads, ...; cell[u] holds the LDS offset of its u-th word in the low
+// (SHIFT 0) or high (SHIFT 16) half, on its set of words that come.  A word
+// whose tag matches carries its value.  false: a neighbour did not answer
+// within ra.limit, or another workgroup gave up.
+template <int U, int SHIFT>
+__device__ __forceinline__ bool receive(const ResidentArgs &ra, const unsigned long long *in_, int tag, float *lds,
+                                        unsigned first, unsigned step, const unsigned (&cell)[U])
+{
     const auto in = gmem(in_);
-    const int th = ra.th, nthr = kTileX * ra.ty, tid = (int)afresh(threadIdx.y * kTileX + threadIdx.x);
-    const int total = ra.words;
-    for (int q0 = tid; q0 < total; q0 += U * nthr) {
-        unsigned wait = 0;
-        int dst[U];
+    unsigned long long since = 0;
+    int tries = 0;
+    unsigned long long w[U];
+    for (;;) {
+        bool ready = true;
 #pragma unroll
-        for (int u = 0; u < U; u++) {
-            const int q = q0 + u * nthr;
-            dst[u] = 0;
-            if (q < 2 * M * kTileX) {
-                const bool above = q >= M * kTileX;
-                const int k = above ? q - M * kTileX : q, l = k / kTileX, x = k % kTileX;
-                if (!above) dst[u] = l < N ? py + (th + l) * spy + x : qy + (th + l - N) * sqy + x;
-                else dst[u] = l < N - 1 ? py + (l - (N - 1)) * spy + x : qy + (l - (N - 1) - N) * sqy + x;
-                if (sides & (above ? kAbove : kBelow)) wait |= 1u << u;
-            } else if (q < total) {
-                const int h = q - 2 * M * kTileX;
-                const bool left = h >= M * th;
-                const int k = left ? h - M * th : h, r = k / M, l = k % M;
-                if (!left) dst[u] = l < N ? px + r * spx + kTileX + l : qx + r * sqx + kTileX + l - N;
-                else dst[u] = l < N - 1 ? px + r * spx + l - (N - 1) : qx + r * sqx + l - (N - 1) - N;
-                if (sides & (left ? kLeft : kRight)) wait |= 1u << u;
+        for (int u = 0; u < U; u++)
+            if (cell[u]) w[u] = __hip_atomic_load(&at(in, afresh(first) + u * step), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (cell[u]) ready &= (int)(w[u] >> 32) == tag;
+        if (ready) break;
+        if ((++tries & 63) == 0 || ra.limit == 0) {
+            const unsigned long long now = wall_clock64();
+            if (since == 0) since = now;
+            if (now - since >= ra.limit) {
+                __hip_atomic_store(gmem(ra.stop), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                return false;
             }
-        }
-        unsigned long long since = 0;
-        int tries = 0;
-        while (wait) {
-            unsigned long long w[U];
-#pragma unroll
-            for (int u = 0; u < U; u++)
-                if (wait & (1u << u))
-                    w[u] = __hip_atomic_load(&at(in, (unsigned)(q0 + u * nthr) * 8u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-#pragma unroll
-            for (int u = 0; u < U; u++)
-                if ((wait & (1u << u)) && (int)(w[u] >> 32) == tag) {
-                    lds[dst[u]] = __uint_as_float((unsigned)w[u]);
-                    wait &= ~(1u << u);
-                }
-            if (wait && ((++tries & 63) == 0 || ra.limit == 0)) {
-                const unsigned long long now = wall_clock64();
-                if (since == 0) since = now;
-                if (now - since >= ra.limit) {
-                    __hip_atomic_store(gmem(ra.stop), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    return false;
-                }
-                if (__hip_atomic_load(gmem(ra.stop), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return false;
-            }
+            if (__hip_atomic_load(gmem(ra.stop), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return false;
         }
     }
+#pragma unroll
+    for (int u = 0; u < U; u++)
+        if (cell[u]) lds[(cell[u] >> SHIFT) & 0xFFFFu] = __uint_as_float((unsigned)w[u]);
     return true;
 }
 
@@ -233,7 +276,6 @@ __global__ __launch_bounds__(kResidentThreads) void k_resident(const ResidentArg
     const int NX = g.NX, NY = g.NY, P = g.pitch;
     const int i = bx * kTileX + tx + 1, j0 = by * th, r0 = ty * R, j = j0 + r0 + 1;  // first row of this thread
     const unsigned c = (unsigned)(j * P + i), e = (unsigned)((j - 1) * NX + (i - 1));  // first cell of this thread
-    const bool fwd = a.sw == 0;
     bool live[R];
 #pragma unroll
     for (int r = 0; r < R; r++) live[r] = i <= NX && j + r <= NY;
@@ -268,59 +310,32 @@ __global__ __launch_bounds__(kResidentThreads) void k_resident(const ResidentArg
         }
     }
 
-    // ---- materials and memory variables
-    float rip[R], rjp[R], m0[R], m1[R], m2[R], m3[R], m4[R], m5[R];
-    float rr[R][L1], pp[R][L1], qq[R][L1];
+    // ---- this thread's words of the inbox: LDS offsets for the stresses (low
+    // half) and the velocities (high half), 0: none
+    constexpr int U = words_per_thread<N, R>();
+    unsigned cell[U];
+    const unsigned word0 = (unsigned)(ty * kTileX + tx), wstep = (unsigned)(kTileX * ra.ty);
 #pragma unroll
-    for (int r = 0; r < R; r++) {
-        const unsigned ci = live[r] ? c + r * P : P + 1u;  // cell (1, 1): every grid has it
-        rip[r] = at(gmem(a.rip), ci * 4u);
-        rjp[r] = at(gmem(a.rjp), ci * 4u);
-        if (L == 0) {
-            m0[r] = at(gmem(a.f), ci * 4u);
-            m1[r] = at(gmem(a.gl), ci * 4u);
-            m2[r] = at(gmem(a.uipjp), ci * 4u);
-        } else {
-            m0[r] = at(gmem(a.mu), ci * 4u);
-            m1[r] = at(gmem(a.pi), ci * 4u);
-            m2[r] = at(gmem(a.muipjp), ci * 4u);
-            m3[r] = at(gmem(a.taus), ci * 4u);
-            m4[r] = at(gmem(a.taup), ci * 4u);
-            m5[r] = at(gmem(a.tausipjp), ci * 4u);
+    for (int u = 0; u < U; u++) {
+        const int q = (int)(word0 + u * wstep);
+        cell[u] = 0;
+        if (q < ra.words) {
+            int side;
+            const unsigned cs = word_cell<N>(q, th, oSYY, kTileX, oSXY, W, oSXX, W, oSXY, W, side);
+            const unsigned cv = word_cell<N>(q, th, oVX, W, oVY, W, oVY, W, oVX, W, side);
+            if (sides & side) cell[u] = cs | cv << 16;
         }
-#pragma unroll
-        for (int l = 0; l < L1; l++) rr[r][l] = pp[r][l] = qq[r][l] = 0.0f;
     }
 
-    // ---- CPML: this column's strip position and profile values
-    int hx = -1;
-    if (i <= g.FW) hx = i - 1;
-    else if (i >= NX - g.FW + 1 && i <= NX) hx = i - NX + 2 * g.FW - 1;
-    float Kx = 1.0f, ax = 0.0f, bxp = 0.0f, Kxh = 1.0f, axh = 0.0f, bxh = 0.0f;
-    if (hx >= 0) {
-        Kx = gmem(g.pml.K_x)[hx]; ax = gmem(g.pml.a_x)[hx]; bxp = gmem(g.pml.b_x)[hx];
-        Kxh = gmem(g.pml.K_xh)[hx]; axh = gmem(g.pml.a_xh)[hx]; bxh = gmem(g.pml.b_xh)[hx];
-    }
-    auto strip_y = [&](int jj) {
-        if (!g.FREE_SURF && jj <= g.FW) return jj - 1;
-        return jj >= NY - g.FW + 1 && jj <= NY ? jj - NY + 2 * g.FW - 1 : -1;
-    };
-    const unsigned hp = hx >= 0 ? (unsigned)((j - 1) * g.px + hx) : 0;  // its first cell in the x strips
-
-    // ---- points at these cells
-    int pi[R], pr[R];
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-        pi[r] = live[r] ? gmem(a.inj.map)[(long)s * a.plane + (e + r * NX)] : -1;
-        pr[r] = live[r] && fwd ? gmem(a.rec.map)[(long)s * a.plane + (e + r * NX)] : -1;
-    }
-    const bool explosive = fwd && gmem(a.explosive)[s] != 0;
-    const bool has_snaps = fwd && has_snap(a);
-    const bool integ = !fwd && a.VELOCITY == 0, energy = a.wacc || a.wacc64;
-    const float scale = L ? (float)(1.0 / (double)g.DH) : g.DT / g.DH;
-    const int NT = a.NT, DTINV = a.DTINV, K_one = g.K_one, fw = g.FW, fs = g.FREE_SURF, vel = a.VELOCITY;
-    const float DT = g.DT, DH = g.DH;
-    float hc[N + 1], eta[L1 + 1], bip[L1 + 1], bjm[L1 + 1], cip[L1 + 1], cjm[L1 + 1];
+    // ---- materials and memory variables.  Up to one row per thread the
+    // buoyancies stay beside their products with DT; else they are read again
+    // where they are needed (snapshots, point forces).
+    constexpr bool kOne = R == 1;
+    float ripk = 0.0f, rjpk = 0.0f, dtx[R], dty[R];
+    float f2[R], gl[R], fip[R];                  // elastic: 2 f, g, fipjp
+    ViscUpdate<L1> vu[R];
+    float rr[R][L1], pp[R][L1], qq[R][L1];
+    float eta[L1 + 1], bip[L1 + 1], bjm[L1 + 1], cip[L1 + 1], cjm[L1 + 1], hc[N + 1];
 #pragma unroll
     for (int m = 1; m <= N; m++) hc[m] = g.hc[m];
 #pragma unroll
@@ -331,244 +346,377 @@ __global__ __launch_bounds__(kResidentThreads) void k_resident(const ResidentArg
         cip[l] = a.cip[l];
         cjm[l] = a.cjm[l];
     }
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const unsigned ci = (live[r] ? c + r * P : P + 1u) * 4u;  // cell (1, 1): every grid has it
+        const float bx_ = at(gmem(a.rip), ci), by_ = at(gmem(a.rjp), ci);
+        if (r == 0) ripk = bx_, rjpk = by_;
+        dtx[r] = g.DT * bx_;
+        dty[r] = g.DT * by_;
+        if (L == 0) {
+            f2[r] = 2.0f * at(gmem(a.f), ci);
+            gl[r] = at(gmem(a.gl), ci);
+            fip[r] = at(gmem(a.uipjp), ci);
+        } else {
+            ViscCell vc;
+            visc_coeffs(L, g.DT, at(gmem(a.mu), ci), at(gmem(a.pi), ci), at(gmem(a.muipjp), ci),
+                        at(gmem(a.taus), ci), at(gmem(a.taup), ci), at(gmem(a.tausipjp), ci), vc);
+            visc_update(vc, eta, vu[r]);
+            if (r == 0 && ty == 0) {
+                float *const sf = lds + D::surface(th) + tx;
+                sf[0] = vc.mu;
+                sf[kTileX] = vc.pi;
+                sf[2 * kTileX] = vc.taus;
+                sf[3 * kTileX] = vc.taup;
+            }
+        }
+#pragma unroll
+        for (int l = 0; l < L1; l++) rr[r][l] = pp[r][l] = qq[r][l] = 0.0f;
+    }
+    auto buoyancies = [&](int r, float &x, float &y) {
+        if constexpr (kOne) {
+            x = ripk;
+            y = rjpk;
+        } else {
+            const auto &b = *afresh(pa);
+            const unsigned ci = (afresh(c) + r * b.g.pitch) * 4u;
+            x = at(gmem(b.rip), ci);
+            y = at(gmem(b.rjp), ci);
+        }
+    };
+
+    // ---- CPML: strip positions of this column and of the rows, and their
+    // profiles, in registers with one row per thread, else in LDS
+    const int fw = g.FW, fs = g.FREE_SURF;
+    auto strip = [&](int k, int n, bool low) {
+        if (low && k <= fw) return k - 1;
+        return k >= n - fw + 1 && k <= n ? k - n + 2 * fw - 1 : -1;
+    };
+    const int hx = strip(i, NX, true);
+    unsigned yrows = 0;  // rows of this thread in a y strip (uniform in a wavefront)
+#pragma unroll
+    for (int r = 0; r < R; r++) yrows |= strip(j + r, NY, !fs) >= 0 ? 1u << r : 0u;
+    const int ylow = fs ? 0 : fw, yshift = 2 * fw - NY;
+    auto strip_row = [&](int jj) { return jj - 1 + (jj > ylow ? yshift : 0); };
+    const bool inx = hx >= 0;
+    Profile xp = {1.0f, 0.0f, 0.0f, 1.0f, 0.0f, 0.0f, 1.0, 1.0}, yp = xp;
+    auto profile = [](int h, const float *K, const float *a_, const float *b, const float *Kh, const float *ah,
+                      const float *bh) {
+        Profile p = {gmem(K)[h], gmem(a_)[h], gmem(b)[h], gmem(Kh)[h], gmem(ah)[h], gmem(bh)[h], 0.0, 0.0};
+        p.rK = 1.0 / (double)p.K;
+        p.rKh = 1.0 / (double)p.Kh;
+        return p;
+    };
+    if (inx) xp = profile(hx, g.pml.K_x, g.pml.a_x, g.pml.b_x, g.pml.K_xh, g.pml.a_xh, g.pml.b_xh);
+    if (kOne && strip(j, NY, !fs) >= 0)
+        yp = profile(strip(j, NY, !fs), g.pml.K_y, g.pml.a_y, g.pml.b_y, g.pml.K_yh, g.pml.a_yh, g.pml.b_yh);
+    float *const xl = lds + D::xprof(th) + tx, *const yl = lds + D::yprof(th);
+    if (!kOne) {
+        if (ty == 0) {
+            xl[0] = xp.K; xl[kTileX] = xp.a; xl[2 * kTileX] = xp.b;
+            xl[3 * kTileX] = xp.Kh; xl[4 * kTileX] = xp.ah; xl[5 * kTileX] = xp.bh;
+            double *const xd2 = (double *)(lds + D::xprof(th) + 6 * kTileX) + tx;
+            xd2[0] = xp.rK;
+            xd2[kTileX] = xp.rKh;
+        }
+        for (int r = ty * kTileX + tx; r < th; r += kTileX * ra.ty) {
+            const int h = strip(j0 + r + 1, NY, !fs);
+            Profile q = {1.0f, 0.0f, 0.0f, 1.0f, 0.0f, 0.0f, 1.0, 1.0};
+            if (h >= 0) q = profile(h, g.pml.K_y, g.pml.a_y, g.pml.b_y, g.pml.K_yh, g.pml.a_yh, g.pml.b_yh);
+            float *const y = yl + 10 * r;
+            y[0] = q.K; y[1] = q.a; y[2] = q.b; y[3] = q.Kh; y[4] = q.ah; y[5] = q.bh;
+            *(double *)(y + 6) = q.rK;
+            *(double *)(y + 8) = q.rKh;
+        }
+    }
+    auto column = [&]() {
+        if constexpr (kOne) return xp;
+        const double *const xd2 = (const double *)(lds + D::xprof(th) + 6 * kTileX) + tx;
+        return Profile{xl[0], xl[kTileX], xl[2 * kTileX], xl[3 * kTileX], xl[4 * kTileX], xl[5 * kTileX], xd2[0],
+                       xd2[kTileX]};
+    };
+    auto row = [&](int r) {
+        if constexpr (kOne) return yp;
+        const float *const y = yl + 10 * (r0 + r);
+        return Profile{y[0], y[1], y[2], y[3], y[4], y[5], *(const double *)(y + 6), *(const double *)(y + 8)};
+    };
+    // byte offsets of the first row's CPML memory
+    const unsigned px4 = (unsigned)g.px * 4u, py4 = (unsigned)g.py * 4u;
+    const unsigned ox = inx ? (unsigned)((j - 1) * g.px + hx) * 4u : 0u, oy = (unsigned)(min(i, NX) - 1) * 4u;
+    const long po = (long)s * a.pss;
+
+    // ---- points at these cells: rows with a source (adjoint: a receiver to
+    // inject at) and rows with a receiver to record, as bits, and the first
+    // point of the first such row; the others are looked up again
+    unsigned inj_rows = 0, rec_rows = 0;
+    int inj_first = -1, rec_first = -1;
+#pragma unroll
+    for (int r = R - 1; r >= 0; r--)
+        if (live[r]) {
+            const int l = gmem(a.inj.map)[(long)s * a.plane + (e + r * NX)];
+            if (l >= 0) inj_rows |= 1u << r, inj_first = l;
+            const int q = a.sw == 0 ? gmem(a.rec.map)[(long)s * a.plane + (e + r * NX)] : -1;
+            if (q >= 0) rec_rows |= 1u << r, rec_first = q;
+        }
+    auto first_of = [&](unsigned rows, int first, const int *map, int r) {
+        if ((rows & ((1u << r) - 1)) == 0) return (int)afresh((unsigned)first);
+        return (int)gmem(map)[(long)s * pa->plane + (afresh(e) + r * NX)];
+    };
+    const bool fwd = a.sw == 0;
+    const bool explosive = fwd && gmem(a.explosive)[s] != 0;
+    const bool has_snaps = fwd && has_snap(a);
+    const bool integ = !fwd && a.VELOCITY == 0, energy = a.wacc != nullptr, energy64 = a.wacc64 != nullptr;
+    const int NT = a.NT, DTINV = a.DTINV, vel = a.VELOCITY;
+    const float DT = g.DT, DH = g.DH, scale = L ? (float)(1.0 / (double)g.DH) : g.DT / g.DH;
+    const double rDH = 1.0 / (double)DH;
+    const float dthalbe = DT / 2.0;
+    // adjoint: vxp1, vyp1 of the correlation; energies of the preconditioner
+    float hvx[R], hvy[R], en[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) hvx[r] = hvy[r] = en[r] = 0.0f;
+    // steps until the next snapshot or correlation, and its slot
+    int until = fwd ? 0 : DTINV - 1;
+    long ks = fwd ? 0 : (long)NT / DTINV - 1;
     __syncthreads();
 
     for (int nt = 1; nt <= NT; nt++) {
-        const bool snap = has_snaps && (nt - 1) % DTINV == 0;
-        const bool corr = !fwd && (NT - nt) % DTINV == 0;
-        const long ks = fwd ? (nt - 1) / DTINV : (NT - nt) / DTINV;
+        const bool mark = until == 0;
+        const bool snap = mark && has_snaps, corr = mark && !fwd;
         const bool rates = snap && vel == 1;
+        float q1 = 0.0f, q2 = 0.0f, q3 = 0.0f, q4 = 0.0f, n1 = 0.0f, n2 = 0.0f, n3 = 0.0f, n4 = 0.0f;
 
         // ================= velocities
-        if (nt > 1 && !receive<N>(ra, in, sides, nt - 1, lds, oSYY, kTileX, oSXY, W, oSXX, W, oSXY, W)) s_stop = 2 * nt;
+        // loads that need no neighbour go ahead of the wait: the samples of a
+        // point, with one row per thread the CPML memory
+        const auto &bv = *afresh(pa);
+        auto load_v = [&](int r) {
+            const auto &b = bv;
+            const unsigned kx = afresh(ox) + r * px4;
+            if (inx && live[r]) n1 = at(gmem(b.psi_sxx_x) + po, kx), n2 = at(gmem(b.psi_sxy_x) + po, kx);
+            if (!(yrows >> r & 1u)) return;
+            const unsigned ky = afresh(oy) + strip_row(j + r) * py4;
+            n3 = at(gmem(b.psi_syy_y) + po, ky), n4 = at(gmem(b.psi_sxy_y) + po, ky);
+        };
+        load_v(0);
+        float s0 = 0.0f, s1 = 0.0f;
+        if (inj_rows) {
+            const long k = (long)(int)afresh((unsigned)inj_first) * NT + nt - 1;
+            s0 = gmem(a.inj.sig)[k];
+            s1 = gmem(a.inj.sig1)[k];
+        }
+        if (nt > 1 && !receive<U, 0>(ra, in, nt - 1, lds, word0 * 8u, wstep * 8u, cell)) s_stop = 2 * nt;
         __syncthreads();
-        if (s_stop && s_stop <= 2 * nt) return;
+        int stop = s_stop;
         {
-            float sxx_x[R], sxy_x[R], sxy_y[R], syy_y[R];
-            {
-                const float *S = SXY + r0 * W + tx, *Y = SYY + r0 * kTileX + tx, *X = SXX + r0 * W + tx;
-                float cy[2 * N + R - 1], cs[2 * N + R - 1];
+            const float *S = SXY + r0 * W + tx, *Y = SYY + r0 * kTileX + tx, *X = SXX + r0 * W + tx;
+            float cy[2 * N + R - 1], cs[2 * N + R - 1];  // cy[k]: sxy row k-N; cs[k]: syy row k-N+1
 #pragma unroll
-                for (int k = 0; k < 2 * N + R - 1; k++) {
-                    cy[k] = S[(k - N) * W];
-                    cs[k] = Y[(k - N + 1) * kTileX];
-                }
-#pragma unroll
-                for (int r = 0; r < R; r++) {
-                    __builtin_amdgcn_sched_barrier(0);
-                    const float *sx = X + r * W, *sy = S + r * W;
-                    sxx_x[r] = hc[1] * (sx[1] - sx[0]);
-                    sxy_x[r] = hc[1] * (cy[N + r] - sy[-1]);
-                    sxy_y[r] = hc[1] * (cy[N + r] - cy[N + r - 1]);
-                    syy_y[r] = hc[1] * (cs[N + r] - cs[N + r - 1]);
-#pragma unroll
-                    for (int m = 2; m <= N; m++) {
-                        sxx_x[r] = sxx_x[r] + hc[m] * (sx[m] - sx[1 - m]);
-                        sxy_x[r] = sxy_x[r] + hc[m] * (sy[m - 1] - sy[-m]);
-                        sxy_y[r] = sxy_y[r] + hc[m] * (cy[N + r + m - 1] - cy[N + r - m]);
-                        syy_y[r] = syy_y[r] + hc[m] * (cs[N + r + m - 1] - cs[N + r - m]);
-                    }
-                }
-            }
-            // CPML: all memory values load before any is stored
-            if (hx >= 0) {
-                const auto &b = *afresh(pa);
-                const auto p1 = gmem(b.psi_sxx_x) + (long)s * b.pss, p2 = gmem(b.psi_sxy_x) + (long)s * b.pss;
-                const unsigned o = afresh(hp), px = b.g.px;
-                float v1[R], v2[R];
-#pragma unroll
-                for (int r = 0; r < R; r++)
-                    if (live[r]) v1[r] = at(p1, (o + r * px) * 4u), v2[r] = at(p2, (o + r * px) * 4u);
-#pragma unroll
-                for (int r = 0; r < R; r++)
-                    if (live[r]) {
-                        v1[r] = bxh * v1[r] + axh * sxx_x[r];
-                        sxx_x[r] = (K_one ? sxx_x[r] : sxx_x[r] / Kxh) + v1[r];
-                        v2[r] = bxp * v2[r] + ax * sxy_x[r];
-                        sxy_x[r] = (K_one ? sxy_x[r] : sxy_x[r] / Kx) + v2[r];
-                        at(p1, (o + r * px) * 4u) = v1[r];
-                        at(p2, (o + r * px) * 4u) = v2[r];
-                    }
+            for (int k = 0; k < 2 * N - 1; k++) {
+                cy[k] = S[(k - N) * W];
+                cs[k] = Y[(k - N + 1) * kTileX];
             }
 #pragma unroll
             for (int r = 0; r < R; r++) {
-                const int h = strip_y(j + r);
-                if (h >= 0 && i <= NX) {
-                    const auto &b = *afresh(pa);
-                    const auto &pm = b.g.pml;
-                    const unsigned o = afresh((unsigned)(i - 1) * 4u);
-                    const auto p1 = gmem(b.psi_syy_y) + (long)s * b.pss + (long)h * b.g.py;
-                    const auto p2 = gmem(b.psi_sxy_y) + (long)s * b.pss + (long)h * b.g.py;
-                    const float v1 = cmem(pm.b_yh)[h] * at(p1, o) + cmem(pm.a_yh)[h] * syy_y[r];
-                    const float v2 = cmem(pm.b_y)[h] * at(p2, o) + cmem(pm.a_y)[h] * sxy_y[r];
-                    syy_y[r] = divK(syy_y[r], pm.K_yh, h, K_one) + v1;
-                    sxy_y[r] = divK(sxy_y[r], pm.K_y, h, K_one) + v2;
-                    at(p1, o) = v1;
-                    at(p2, o) = v2;
-                }
-            }
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                __builtin_amdgcn_sched_barrier(0);
+                if (!kOne) __builtin_amdgcn_sched_barrier(0);
+                q1 = n1, q2 = n2, q3 = n3, q4 = n4;
+                if (r + 1 < R) load_v(r + 1);
+                cy[2 * N - 1 + r] = S[(N - 1 + r) * W];
+                cs[2 * N - 1 + r] = Y[(N + r) * kTileX];
+                // one row per thread: every LDS value is on its way before the first is
+                // used (more rows have no registers to spare for it)
                 const int o = (r0 + r) * W + tx;
-                const float vx0 = VX[o], vy0 = VY[o];
-                float vx = vel_new(vx0, DT, rip[r], sxx_x[r] + sxy_y[r], DH);
-                float vy = vel_new(vy0, DT, rjp[r], sxy_x[r] + syy_y[r], DH);
-                if (pi[r] >= 0) {
-                    const auto &b = *afresh(pa);
-                    for (int l = pi[r]; l >= 0; l = gmem(b.inj.next)[l]) inject(b, l, nt, rip[r], rjp[r], vx, vy);
+                float sx[2 * N], sy[2 * N];  // columns i-N+1 .. i+N and i-N .. i+N-1
+#pragma unroll
+                for (int k = 0; k < 2 * N; k++) {
+                    sx[k] = X[r * W + k - N + 1];
+                    sy[k] = k == N ? 0.0f : S[r * W + k - N];
                 }
-                if (!live[r]) vx = vy = 0.0f;
+                const float vx0 = VX[o], vy0 = VY[o];
+                if (kOne) __builtin_amdgcn_sched_barrier(0);
+                if (r == 0 && stop && stop <= 2 * nt) return;
+                sy[N] = cy[N + r];
+                float sxx_x = hc[1] * (sx[N] - sx[N - 1]);
+                float sxy_x = hc[1] * (sy[N] - sy[N - 1]);
+                float sxy_y = hc[1] * (cy[N + r] - cy[N + r - 1]);
+                float syy_y = hc[1] * (cs[N + r] - cs[N + r - 1]);
+#pragma unroll
+                for (int m = 2; m <= N; m++) {
+                    sxx_x = sxx_x + hc[m] * (sx[N + m - 1] - sx[N - m]);
+                    sxy_x = sxy_x + hc[m] * (sy[N + m - 1] - sy[N - m]);
+                    sxy_y = sxy_y + hc[m] * (cy[N + r + m - 1] - cy[N + r - m]);
+                    syy_y = syy_y + hc[m] * (cs[N + r + m - 1] - cs[N + r - m]);
+                }
+                if (inx && live[r]) {
+                    const Profile x = column();
+                    const unsigned kx = afresh(ox) + r * px4;
+                    absorb(sxx_x, q1, x.Kh, x.rKh, x.ah, x.bh, sxy_x, q2, x.K, x.rK, x.a, x.b);
+                    at(gmem(bv.psi_sxx_x) + po, kx) = q1;
+                    at(gmem(bv.psi_sxy_x) + po, kx) = q2;
+                }
+                if ((yrows >> r & 1u) && i <= NX) {
+                    const Profile y = row(r);
+                    const unsigned ky = afresh(oy) + strip_row(j + r) * py4;
+                    absorb(syy_y, q3, y.Kh, y.rKh, y.ah, y.bh, sxy_y, q4, y.K, y.rK, y.a, y.b);
+                    at(gmem(bv.psi_syy_y) + po, ky) = q3;
+                    at(gmem(bv.psi_sxy_y) + po, ky) = q4;
+                }
+                const float sumx = sxx_x + sxy_y, sumy = sxy_x + syy_y;
+                float vx = dtx[r] * sumx, vy = dty[r] * sumy;  // vel_new
+                div_by2(vx, vy, DH, DH, rDH, rDH);
+                vx = vx0 + vx;
+                vy = vy0 + vy;
+                if (inj_rows >> r & 1u) {
+                    const auto &b = *afresh(pa);
+                    float rip, rjp;
+                    buoyancies(r, rip, rjp);
+                    int l = first_of(inj_rows, inj_first, b.inj.map, r);
+                    if ((inj_rows & ((1u << r) - 1)) == 0) {
+                        inject_values(b, l, s0, s1, rip, rjp, vx, vy);
+                        l = gmem(b.inj.next)[l];
+                    }
+                    for (; l >= 0; l = gmem(b.inj.next)[l]) inject(b, l, nt, rip, rjp, vx, vy);
+                }
+                if (i > NX || (kOne ? j : afresh_uniform(j)) + r > NY) vx = vy = 0.0f;
                 VX[o] = vx;
                 VY[o] = vy;
-                send_y<N>(ra, sides, up + ra.words, dn + ra.words, r0 + r, (int)afresh(tx), vx, vy, nt);
-                XDest xv = xd;  // the velocity half of the inboxes
-                xv.p += xd.p >= 0 ? ra.words : 0;
-                xv.q += xd.q >= 0 ? ra.words : 0;
-                send_x<N>(ra, xv, r, vy, vx, nt);
+                send_y<N>(ra, sides, up + ra.words, dn + ra.words, (kOne ? r0 : afresh_uniform(r0)) + r, (int)afresh((unsigned)tx), vx, vy, nt);
+                send_x<N>(ra, xd, ra.words, r, vy, vx, nt);
+                if (!fwd) {
+                    if (integ) {
+                        hvx[r] += vx0 * DT;
+                        hvy[r] += vy0 * DT;
+                    } else if (corr) {
+                        hvx[r] = vx0;
+                        hvy[r] = vy0;
+                    }
+                }
+                if (energy) en[r] += ((vx * vx) + (vy * vy));
                 if (snap) {
                     const auto &b = *afresh(pa);
-                    const float acc[2] = {vel_rate(rip[r], sxx_x[r] + sxy_y[r], DH),
-                                          vel_rate(rjp[r], sxy_x[r] + syy_y[r], DH)};
+                    float rip, rjp;
+                    buoyancies(r, rip, rjp);
+                    const float acc[2] = {vel_rate(rip, sumx, afresh(DH)), vel_rate(rjp, sumy, afresh(DH))};
                     float *const keep[2] = {b.vxp1, b.vyp1};
                     res_snap_put<2>(b, s, 0, ks, afresh(e) + r * NX, afresh(c) + r * P, live[r], r0 + r, acc, keep,
                                     maxima);
                 }
-                if (!live[r]) continue;
-                if (integ || corr) {
+                if (energy64 && live[r]) {
                     const auto &b = *afresh(pa);
-                    const auto qx = gmem(b.vxp1) + (long)s * b.ws, qy = gmem(b.vyp1) + (long)s * b.ws;
-                    const unsigned cr = (afresh(c) + r * P) * 4u;
-                    if (integ) {
-                        at(qx, cr) += vx0 * DT;
-                        at(qy, cr) += vy0 * DT;
-                    } else {
-                        at(qx, cr) = vx0;
-                        at(qy, cr) = vy0;
-                    }
-                }
-                if (energy) {
-                    const auto &b = *afresh(pa);
-                    const unsigned er = afresh(e) + r * NX;
-                    if (b.wacc64) {
-                        const auto Wd = gmem(b.wacc64) + (long)s * b.wacs;
-                        at(Wd, er * 8u) += ((double)vx * (double)vx) + ((double)vy * (double)vy);
-                    } else {
-                        const auto Wf = gmem(b.wacc) + (long)s * b.wacs;
-                        at(Wf, er * 4u) += ((vx * vx) + (vy * vy));
-                    }
+                    const auto Wd = gmem(b.wacc64) + (long)s * b.wacs;
+                    at(Wd, (afresh(e) + r * NX) * 8u) += ((double)vx * (double)vx) + ((double)vy * (double)vy);
                 }
             }
             if (snap) {
                 const auto &b = *afresh(pa);
                 float *const keep[2] = {b.vxp1, b.vyp1};
-                res_snap_encode<2, R>(b, s, 0, ks, e, c, i, j, r0, bx, keep, maxima);
+                res_snap_encode<2, R>(b, s, 0, ks, afresh(e), afresh(c), i, j, r0, bx, keep, maxima);
             }
         }
 
         // ================= stresses
-        if (!receive<N>(ra, in + ra.words, sides, nt, lds, oVX, W, oVY, W, oVY, W, oVX, W)) s_stop = 2 * nt + 1;
+        const auto &bs = *afresh(pa);
+        auto load_s = [&](int r) {
+            const auto &b = bs;
+            const unsigned kx = afresh(ox) + r * px4;
+            if (inx && live[r]) n1 = at(gmem(b.psi_vxx) + po, kx), n2 = at(gmem(b.psi_vyx) + po, kx);
+            if (!(yrows >> r & 1u)) return;
+            const unsigned ky = afresh(oy) + strip_row(j + r) * py4;
+            n3 = at(gmem(b.psi_vyy) + po, ky), n4 = at(gmem(b.psi_vxy) + po, ky);
+        };
+        load_s(0);
+        float amp = 0.0f;
+        if (explosive && inj_rows)
+            amp = explosive_amp(a.exp.sig + (long)(int)afresh((unsigned)inj_first) * NT - 1, nt, NT, afresh(DH));
+        if (!receive<U, 16>(ra, in + ra.words, nt, lds, word0 * 8u, wstep * 8u, cell)) s_stop = 2 * nt + 1;
         __syncthreads();
-        if (s_stop && s_stop <= 2 * nt + 1) return;
+        stop = s_stop;
         {
-            float vxx[R], vyx[R], vxy[R], vyy[R];
-            {
-                const float *X = VX + r0 * W + tx, *Y = VY + r0 * W + tx;
-                float cx[2 * N + R - 1], cy[2 * N + R - 1];  // cx[k]: vx row k-N+1; cy[k]: vy row k-N
+            const float *X = VX + r0 * W + tx, *Y = VY + r0 * W + tx;
+            float cx[2 * N + R - 1], cy[2 * N + R - 1];  // cx[k]: vx row k-N+1; cy[k]: vy row k-N
 #pragma unroll
-                for (int k = 0; k < 2 * N + R - 1; k++) {
-                    cx[k] = X[(k - N + 1) * W];
-                    cy[k] = Y[(k - N) * W];
-                }
-#pragma unroll
-                for (int r = 0; r < R; r++) {
-                    __builtin_amdgcn_sched_barrier(0);
-                    const float *vx = X + r * W, *vy = Y + r * W;
-                    vxx[r] = hc[1] * (cx[N - 1 + r] - vx[-1]);
-                    vyx[r] = hc[1] * (vy[1] - cy[N + r]);
-                    vxy[r] = hc[1] * (cx[N + r] - cx[N - 1 + r]);
-                    vyy[r] = hc[1] * (cy[N + r] - cy[N + r - 1]);
-#pragma unroll
-                    for (int m = 2; m <= N; m++) {
-                        vxx[r] = vxx[r] + hc[m] * (vx[m - 1] - vx[-m]);
-                        vyx[r] = vyx[r] + hc[m] * (vy[m] - vy[1 - m]);
-                        vxy[r] = vxy[r] + hc[m] * (cx[N - 1 + r + m] - cx[N + r - m]);
-                        vyy[r] = vyy[r] + hc[m] * (cy[N + r + m - 1] - cy[N + r - m]);
-                    }
-                    vxx[r] = vxx[r] * scale;
-                    vyx[r] = vyx[r] * scale;
-                    vxy[r] = vxy[r] * scale;
-                    vyy[r] = vyy[r] * scale;
-                }
-            }
-            if (hx >= 0) {
-                const auto &b = *afresh(pa);
-                const auto p1 = gmem(b.psi_vxx) + (long)s * b.pss, p2 = gmem(b.psi_vyx) + (long)s * b.pss;
-                const unsigned o = afresh(hp), px = b.g.px;
-                float v1[R], v2[R];
-#pragma unroll
-                for (int r = 0; r < R; r++)
-                    if (live[r]) v1[r] = at(p1, (o + r * px) * 4u), v2[r] = at(p2, (o + r * px) * 4u);
-#pragma unroll
-                for (int r = 0; r < R; r++)
-                    if (live[r]) {
-                        v1[r] = bxp * v1[r] + ax * vxx[r];
-                        vxx[r] = (K_one ? vxx[r] : vxx[r] / Kx) + v1[r];
-                        v2[r] = bxh * v2[r] + axh * vyx[r];
-                        vyx[r] = (K_one ? vyx[r] : vyx[r] / Kxh) + v2[r];
-                        at(p1, (o + r * px) * 4u) = v1[r];
-                        at(p2, (o + r * px) * 4u) = v2[r];
-                    }
+            for (int k = 0; k < 2 * N - 1; k++) {
+                cx[k] = X[(k - N + 1) * W];
+                cy[k] = Y[(k - N) * W];
             }
 #pragma unroll
             for (int r = 0; r < R; r++) {
-                const int h = strip_y(j + r);
-                if (h >= 0 && i <= NX) {
-                    const auto &b = *afresh(pa);
-                    const auto &pm = b.g.pml;
-                    const unsigned o = afresh((unsigned)(i - 1) * 4u);
-                    const auto p1 = gmem(b.psi_vyy) + (long)s * b.pss + (long)h * b.g.py;
-                    const auto p2 = gmem(b.psi_vxy) + (long)s * b.pss + (long)h * b.g.py;
-                    const float v1 = cmem(pm.b_y)[h] * at(p1, o) + cmem(pm.a_y)[h] * vyy[r];
-                    const float v2 = cmem(pm.b_yh)[h] * at(p2, o) + cmem(pm.a_yh)[h] * vxy[r];
-                    vyy[r] = divK(vyy[r], pm.K_y, h, K_one) + v1;
-                    vxy[r] = divK(vxy[r], pm.K_yh, h, K_one) + v2;
-                    at(p1, o) = v1;
-                    at(p2, o) = v2;
-                }
-            }
+                if (!kOne) __builtin_amdgcn_sched_barrier(0);
+                q1 = n1, q2 = n2, q3 = n3, q4 = n4;
+                if (r + 1 < R) load_s(r + 1);
+                cx[2 * N - 1 + r] = X[(N + r) * W];
+                cy[2 * N - 1 + r] = Y[(N - 1 + r) * W];
+                const int o = (r0 + r) * W + tx, oyy = (r0 + r) * kTileX + tx;
+                float xv[2 * N], yv[2 * N];  // vx at columns i-N .. i+N-1, vy at i-N+1 .. i+N
 #pragma unroll
-            for (int r = 0; r < R; r++) {
-                __builtin_amdgcn_sched_barrier(0);
-                const int o = (r0 + r) * W + tx, oy = (r0 + r) * kTileX + tx;
-                float sxx = SXX[o], syy = SYY[oy], sxy = SXY[o];
+                for (int k = 0; k < 2 * N; k++) {
+                    xv[k] = k == N ? 0.0f : X[r * W + k - N];
+                    yv[k] = k == N - 1 ? 0.0f : Y[r * W + k - N + 1];
+                }
+                float sxx = SXX[o], syy = SYY[oyy], sxy = SXY[o];
+                if (kOne) __builtin_amdgcn_sched_barrier(0);
+                if (r == 0 && stop && stop <= 2 * nt + 1) return;
+                xv[N] = cx[N - 1 + r];
+                yv[N - 1] = cy[N + r];
+                float vxx = hc[1] * (xv[N] - xv[N - 1]);
+                float vyx = hc[1] * (yv[N] - yv[N - 1]);
+                float vxy = hc[1] * (cx[N + r] - cx[N - 1 + r]);
+                float vyy = hc[1] * (cy[N + r] - cy[N + r - 1]);
+#pragma unroll
+                for (int m = 2; m <= N; m++) {
+                    vxx = vxx + hc[m] * (xv[N + m - 1] - xv[N - m]);
+                    vyx = vyx + hc[m] * (yv[N + m - 1] - yv[N - m]);
+                    vxy = vxy + hc[m] * (cx[N - 1 + r + m] - cx[N + r - m]);
+                    vyy = vyy + hc[m] * (cy[N + r + m - 1] - cy[N + r - m]);
+                }
+                vxx = vxx * scale;
+                vyx = vyx * scale;
+                vxy = vxy * scale;
+                vyy = vyy * scale;
+                if (inx && live[r]) {
+                    const Profile x = column();
+                    const unsigned kx = afresh(ox) + r * px4;
+                    absorb(vxx, q1, x.K, x.rK, x.a, x.b, vyx, q2, x.Kh, x.rKh, x.ah, x.bh);
+                    at(gmem(bs.psi_vxx) + po, kx) = q1;
+                    at(gmem(bs.psi_vyx) + po, kx) = q2;
+                }
+                if ((yrows >> r & 1u) && i <= NX) {
+                    const Profile y = row(r);
+                    const unsigned ky = afresh(oy) + strip_row(j + r) * py4;
+                    absorb(vyy, q3, y.K, y.rK, y.a, y.b, vxy, q4, y.Kh, y.rKh, y.ah, y.bh);
+                    at(gmem(bs.psi_vyy) + po, ky) = q3;
+                    at(gmem(bs.psi_vxy) + po, ky) = q4;
+                }
                 float ux = 0.0f, uy = 0.0f, uxy = 0.0f;
-                ViscCell vc;
                 if (L == 0) {
-                    if (rates) rates_elastic(m0[r], m1[r], m2[r], DT, vxx[r], vyx[r], vxy[r], vyy[r], ux, uy, uxy);
-                    stress_elastic(m0[r], m1[r], m2[r], vxx[r], vyx[r], vxy[r], vyy[r], sxx, syy, sxy);
+                    if (rates)
+                        rates_elastic(0.5f * afresh(f2[r]), afresh(gl[r]), afresh(fip[r]), afresh(DT), vxx, vyx, vxy,
+                                      vyy, ux, uy, uxy);
+                    stress_elastic(f2[r], gl[r], fip[r], vxx, vyx, vxy, vyy, sxx, syy, sxy);
                 } else {
-                    // opaque, so that the products formed from them stay out of
-                    // the registers between steps
-                    asm volatile("" : "+v"(m0[r]), "+v"(m1[r]), "+v"(m2[r]), "+v"(m3[r]), "+v"(m4[r]), "+v"(m5[r]));
-                    visc_coeffs(L, DT, m0[r], m1[r], m2[r], m3[r], m4[r], m5[r], vc);
-                    stress_visc<L1>(vc, eta, bip, bjm, cip, cjm, DT, vxx[r], vyx[r], vxy[r], vyy[r], sxx,
-                                    syy, sxy, rr[r], pp[r], qq[r], rates, ux, uy, uxy);
+                    ViscUpdate<L1> v = vu[r];
+                    if (!kOne) v.f2 = afresh(v.f2);  // its FP64 value need not stay in registers
+                    stress_visc(v, bip, bjm, cip, cjm, dthalbe, afresh(DT), vxx, vyx, vxy, vyy, sxx, syy, sxy, rr[r], pp[r], qq[r],
+                                rates, ux, uy, uxy);
                 }
-                if (explosive && pi[r] >= 0) {
+                if (explosive && (inj_rows >> r & 1u)) {
                     const auto &b = *afresh(pa);
-                    for (int l = pi[r]; l >= 0; l = gmem(b.exp.next)[l]) {
-                        const float amp = explosive_amp(b.exp.sig + (long)l * NT - 1, nt, NT, DH);
-                        sxx = add_half(sxx, amp);
-                        syy = add_half(syy, amp);
+                    int l = first_of(inj_rows, inj_first, b.inj.map, r);
+                    float x = amp;
+                    if (inj_rows & ((1u << r) - 1)) x = explosive_amp(b.exp.sig + (long)l * NT - 1, nt, NT, afresh(DH));
+                    for (;;) {
+                        sxx = add_half(sxx, x);
+                        syy = add_half(syy, x);
+                        l = gmem(b.exp.next)[l];
+                        if (l < 0) break;
+                        x = explosive_amp(b.exp.sig + (long)l * NT - 1, nt, NT, afresh(DH));
                     }
                 }
-                const int jr = j + r;  // row of the grid
+                const int jr = (kOne ? j : afresh_uniform(j)) + r;  // row of the grid
                 if (fs && by == 0 && jr <= N + 1) {
                     // free surface: the mirrored rows above, and row 1 itself
                     if (jr >= 2) SYY[(2 - jr - 1) * kTileX + tx] = live[r] ? -syy : 0.0f;
                     if (jr <= N) SXY[(1 - jr - 1) * W + tx] = live[r] ? -sxy : 0.0f;
-                    if (jr == 1) {
+                    if (r == 0 && jr == 1) {
                         syy = 0.0f;
                         if (rates) uy = 0.0f;
                         if (L) {
@@ -582,29 +730,33 @@ __global__ __launch_bounds__(kResidentThreads) void k_resident(const ResidentArg
                             dx += hc[m] * (vx[m - 1] - vx[-m]);
                             dy += hc[m] * (vy[(m - 1) * W] - vy[-m * W]);
                         }
-                        const float dh24 = 1.0 / (double)DH;
+                        const float dh24 = 1.0 / (double)afresh(DH);
                         dx *= dh24;
                         dy *= dh24;
-                        if (hx >= 0) {
+                        if (inx) {
                             const auto &b = *afresh(pa);
                             const auto ps = gmem(b.psi_vxxs) + (long)s * b.pss + (unsigned)hx;
-                            const float v = bxp * *ps + ax * dx;
-                            dx = (K_one ? dx : dx / Kx) + v;
+                            const Profile x = column();
+                            float v = *ps;
+                            v = x.b * v + x.a * dx;
+                            dx = div_by(dx, x.K, x.rK) + v;
                             *ps = v;
                         }
-                        if (L == 0)
-                            surface_elastic_update((float)((double)m0[r] * 2.0), m1[r], DT, dx, dy, sxx, rates, ux);
-                        else
-                            surface_visc_update<L1>(vc.mu, vc.pi, vc.taus, vc.taup, eta, DT, dx, dy, sxx, pp[r],
-                                                    rates, ux);
+                        if (L == 0) {
+                            surface_elastic_update(afresh(f2[r]), afresh(gl[r]), DT, dx, dy, sxx, rates, ux);
+                        } else {
+                            const float *const sf = lds + D::surface(th) + tx;
+                            surface_visc_update<L1>(sf[0], sf[kTileX], sf[2 * kTileX], sf[3 * kTileX], eta, DT, dx,
+                                                    dy, sxx, pp[r], rates, ux);
+                        }
                     }
                 }
-                if (!live[r]) sxx = syy = sxy = 0.0f;
+                if (i > NX || jr > NY) sxx = syy = sxy = 0.0f;
                 SXX[o] = sxx;
-                SYY[oy] = syy;
+                SYY[oyy] = syy;
                 SXY[o] = sxy;
-                send_y<N>(ra, sides, up, dn, r0 + r, (int)afresh(tx), syy, sxy, nt);
-                send_x<N>(ra, xd, r, sxx, sxy, nt);
+                send_y<N>(ra, sides, up, dn, (kOne ? r0 : afresh_uniform(r0)) + r, (int)afresh((unsigned)tx), syy, sxy, nt);
+                send_x<N>(ra, xd, 0, r, sxx, sxy, nt);
                 if (snap) {
                     const auto &b = *afresh(pa);
                     const float u[3] = {vel ? ux : sxx, vel ? uy : syy, vel ? uxy : sxy};
@@ -612,9 +764,9 @@ __global__ __launch_bounds__(kResidentThreads) void k_resident(const ResidentArg
                     res_snap_put<3>(b, s, 2, ks, afresh(e) + r * NX, afresh(c) + r * P, live[r], r0 + r, u, keep,
                                     maxima + 2 * th);
                 }
-                if (pr[r] >= 0) {
+                if (rec_rows >> r & 1u) {
                     const auto &b = *afresh(pa);
-                    for (int l = pr[r]; l >= 0; l = gmem(b.rec.next)[l]) {
+                    for (int l = first_of(rec_rows, rec_first, b.rec.map, r); l >= 0; l = gmem(b.rec.next)[l]) {
                         gmem(b.seis_vx)[(long)l * NT + nt - 1] = VX[o];
                         gmem(b.seis_vy)[(long)l * NT + nt - 1] = VY[o];
                     }
@@ -627,33 +779,39 @@ __global__ __launch_bounds__(kResidentThreads) void k_resident(const ResidentArg
             if (snap) {
                 const auto &b = *afresh(pa);
                 float *const keep[3] = {b.ux, b.uy, b.uxy};
-                res_snap_encode<3, R>(b, s, 2, ks, e, c, i, j, r0, bx, keep, maxima + 2 * th);
+                res_snap_encode<3, R>(b, s, 2, ks, afresh(e), afresh(c), i, j, r0, bx, keep, maxima + 2 * th);
             }
             if (corr) {
-#pragma unroll 1
+#pragma unroll
                 for (int r = 0; r < R; r++) {
-                    if (i > NX || j + r > NY) break;
+                    if (!live[r]) break;
+                    if (!kOne) __builtin_amdgcn_sched_barrier(0);
                     const auto &b = *afresh(pa);
-                    const int o = (r0 + r) * W + tx, oy = (r0 + r) * kTileX + tx;
-                    const unsigned cr = (afresh(c) + r * P) * 4u, ei = afresh(e) + r * NX, er = ei * 4u;
+                    const int o = (r0 + r) * W + tx, oyy = (r0 + r) * kTileX + tx;
+                    const unsigned ei = afresh(e) + r * NX, er = ei * 4u;
                     const int blk = (j + r - 1) / kTileY * b.nbx + bx;
-                    const long wco = (long)s * b.wcs, wo = (long)s * b.ws;
+                    const long wco = (long)s * b.wcs;
                     const auto Wr = gmem(b.wc_rho) + wco, Wl = gmem(b.wc) + wco, Wu = gmem(b.wc_u) + wco;
                     float wr = at(Wr, er), w = at(Wl, er), wu = at(Wu, er);
-                    correlate_cell(at(gmem(b.vxp1) + wo, cr), at(gmem(b.vyp1) + wo, cr), SXX[o], SYY[oy], SXY[o],
-                                   res_snap_load(b, s, 0, ks, ei, blk), res_snap_load(b, s, 1, ks, ei, blk),
-                                   res_snap_load(b, s, 2, ks, ei, blk), res_snap_load(b, s, 3, ks, ei, blk),
-                                   res_snap_load(b, s, 4, ks, ei, blk), at(gmem(b.muss), er), at(gmem(b.lamss), er),
-                                   at(gmem(b.vs_i), er) > 0.0f, wr, w, wu);
+                    correlate_cell(hvx[r], hvy[r], SXX[o], SYY[oyy], SXY[o], res_snap_load(b, s, 0, ks, ei, blk),
+                                   res_snap_load(b, s, 1, ks, ei, blk), res_snap_load(b, s, 2, ks, ei, blk),
+                                   res_snap_load(b, s, 3, ks, ei, blk), res_snap_load(b, s, 4, ks, ei, blk),
+                                   at(gmem(b.muss), er), at(gmem(b.lamss), er), at(gmem(b.vs_i), er) > 0.0f, wr, w,
+                                   wu);
                     at(Wr, er) = wr;
                     at(Wl, er) = w;
                     at(Wu, er) = wu;
                 }
             }
         }
+        if (mark) {
+            until = DTINV;
+            ks += fwd ? 1 : -1;
+        }
+        until--;
     }
 
-    // ---- the final wavefields, where the two-kernel step keeps them
+    // ---- the final wavefields, where the two-kernel step keeps them, and the energies
 #pragma unroll
     for (int r = 0; r < R; r++)
         if (live[r]) {
@@ -665,6 +823,7 @@ __global__ __launch_bounds__(kResidentThreads) void k_resident(const ResidentArg
             at(gmem(a.sxx) + wo, cr * 4u) = SXX[o];
             at(gmem(a.syy) + wo, cr * 4u) = SYY[(r0 + r) * kTileX + tx];
             at(gmem(a.sxy) + wo, cr * 4u) = SXY[o];
+            if (energy) at(gmem(a.wacc) + (long)s * a.wacs, (e + r * NX) * 4u) = en[r];
         }
 }
 

@@ -140,6 +140,8 @@ ResidentPlan resident_plan(const StepGeom &g, int L, int nslots, int snap_prec, 
     if (g.BOUNDARY || most == 0 || nslots < 1 || (long)nbx * nslots > ncu) return p;
     const int across = ncu / (nbx * nslots);  // tile rows per slot that fit
     int th = std::max((g.NY + across - 1) / across, g.N + (g.FREE_SURF ? 1 : 0));
+    const int line = 2 * (2 * g.N - 1);
+    while (line * (kTileX + th) > kWordsPerThread * kTileX * th) th++;
     for (int rows = 1; rows <= most; rows++) {
         int ty = (th + rows - 1) / rows;
         // the scales of 16-bit snapshots belong to 64x8 tiles

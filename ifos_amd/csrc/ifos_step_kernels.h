@@ -415,7 +415,7 @@ __device__ __forceinline__ void str_cell(const StepArgs &a, int s, int blk, int 
         sxy = gmem(a.sxy)[wo + c];
         if (L == 0) {
             if (rates) rates_elastic(M.fe, M.ge, M.fipjp, g.DT, vxx, vyx, vxy, vyy, ux, uy, uxy);
-            stress_elastic(M.fe, M.ge, M.fipjp, vxx, vyx, vxy, vyy, sxx, syy, sxy);
+            stress_elastic(2.0f * M.fe, M.ge, M.fipjp, vxx, vyx, vxy, vyy, sxx, syy, sxy);
         } else {
 #pragma unroll
             for (int l = 0; l < L; l++) {
@@ -423,8 +423,10 @@ __device__ __forceinline__ void str_cell(const StepArgs &a, int s, int blk, int 
                 pp[l] = gmem(a.r)[wo + mv_index(c, L + l, 3 * L)];
                 qq[l] = gmem(a.r)[wo + mv_index(c, 2 * L + l, 3 * L)];
             }
-            stress_visc<(L > 0 ? L : 1)>(M.vc, a.eta, a.bip, a.bjm, a.cip, a.cjm, g.DT, vxx, vyx, vxy, vyy, sxx, syy,
-                                       sxy, rr, pp, qq, rates, ux, uy, uxy);
+            ViscUpdate<(L > 0 ? L : 1)> vu;
+            visc_update(M.vc, a.eta, vu);
+            stress_visc(vu, a.bip, a.bjm, a.cip, a.cjm, g.DT / 2.0, g.DT, vxx, vyx, vxy, vyy, sxx, syy, sxy, rr, pp, qq, rates,
+                        ux, uy, uxy);
         }
         // explosive sources of this cell, applied after the stress update
         // and before the free surface (src/IFOS2D.c:1758-1773)
@@ -778,7 +780,7 @@ __global__ __launch_bounds__(512) void k_fused_step(const StepArgs *__restrict__
             sxy = st.sxy[ty + 2 * N][tx + 2 * N];
             if (L == 0) {
                 if (rates) rates_elastic(M.fe, M.ge, M.fipjp, g.DT, vxx, vyx, vxy, vyy, ux, uy, uxy);
-                stress_elastic(M.fe, M.ge, M.fipjp, vxx, vyx, vxy, vyy, sxx, syy, sxy);
+                stress_elastic(2.0f * M.fe, M.ge, M.fipjp, vxx, vyx, vxy, vyy, sxx, syy, sxy);
             } else {
 #pragma unroll
                 for (int l = 0; l < L; l++) {
@@ -786,8 +788,10 @@ __global__ __launch_bounds__(512) void k_fused_step(const StepArgs *__restrict__
                     pp[l] = gmem(a.r)[wo + mv_index(c, L + l, 3 * L)];
                     qq[l] = gmem(a.r)[wo + mv_index(c, 2 * L + l, 3 * L)];
                 }
-                stress_visc<(L > 0 ? L : 1)>(M.vc, a.eta, a.bip, a.bjm, a.cip, a.cjm, g.DT, vxx, vyx, vxy, vyy, sxx,
-                                           syy, sxy, rr, pp, qq, rates, ux, uy, uxy);
+                ViscUpdate<(L > 0 ? L : 1)> vu;
+                visc_update(M.vc, a.eta, vu);
+                stress_visc(vu, a.bip, a.bjm, a.cip, a.cjm, g.DT / 2.0, g.DT, vxx, vyx, vxy, vyy, sxx, syy, sxy, rr, pp, qq,
+                            rates, ux, uy, uxy);
             }
             for (int l = ex; l >= 0; l = gmem(a.exp.next)[l]) {
                 const float amp = explosive_amp(a.exp.sig + (long)l * a.NT - 1, nt, a.NT, g.DH);

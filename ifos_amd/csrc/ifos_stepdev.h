@@ -136,14 +136,14 @@ __device__ __forceinline__ int first_point(const StepArgs &a, const PointMap &p,
     return any ? gmem(p.map)[(long)s * a.plane + e] : -1;
 }
 
-// point force (forward) or residual injection (adjoint) of point l at step nt
-// (A: the argument block through a plain or a constant-space reference)
+// point force (forward) or residual injection (adjoint) of point l at step
+// nt, whose samples are s0, s1 (A: the argument block through a plain or a
+// constant-space reference)
 template <class A>
-__device__ __forceinline__ void inject(A &a, int l, int nt, float rip, float rjp, float &vx, float &vy)
+__device__ __forceinline__ void inject_values(A &a, int l, float s0, float s1, float rip, float rjp, float &vx,
+                                              float &vy)
 {
     const auto &g = a.g;
-    const float s0 = gmem(a.inj.sig)[(long)l * a.NT + nt - 1];
-    const float s1 = gmem(a.inj.sig1)[(long)l * a.NT + nt - 1];
     if (a.sw == 0) {
         const int type = gmem(a.inj.type)[l];
         if (type == 2) vx += (g.DT * rip * s1) / (g.DH * g.DH);
@@ -157,6 +157,13 @@ __device__ __forceinline__ void inject(A &a, int l, int nt, float rip, float rjp
         if (a.ADJOINT_TYPE == 2) vy += s1;
         if (a.ADJOINT_TYPE == 3) vx += s0;
     }
+}
+
+template <class A>
+__device__ __forceinline__ void inject(A &a, int l, int nt, float rip, float rjp, float &vx, float &vy)
+{
+    inject_values(a, l, gmem(a.inj.sig)[(long)l * a.NT + nt - 1], gmem(a.inj.sig1)[(long)l * a.NT + nt - 1], rip, rjp,
+                  vx, vy);
 }
 
 // ---------------------------------------------------------------------------

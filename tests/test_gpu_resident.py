@@ -55,7 +55,7 @@ def test_resident_equals_per_step_kernels(gpu_lib, c, kw):
 
 
 @pytest.mark.parametrize("c", [dict(NX=64, NY=4096, L=0), dict(NX=64, NY=4097, L=2), dict(NX=1024, NY=256, L=1),
-                               dict(NX=1024, NY=257, L=0), dict(NX=900, NY=530, L=0), dict(NX=960, NY=768, L=0)],
+                               dict(NX=1024, NY=257, L=0), dict(NX=900, NY=530, L=0), dict(NX=900, NY=700, L=2), dict(NX=960, NY=1024, L=0)],
                          ids=lambda c: f"{c['NX']}x{c['NY']}_L{c['L']}")
 @pytest.mark.parametrize("order", [2, 8])
 def test_resident_large_tiles(gpu_lib, c, order):
