@@ -7,7 +7,7 @@ namespace ifos {
 template void vel_n<4>(const StepArgs &a, const StepArgs *da, const LaunchShape &ls, int k, hipStream_t s);
 template void str_n<4>(const StepArgs &a, const StepArgs *da, const LaunchShape &ls, int k, hipStream_t s);
 template void fused_n<4>(const StepArgs &a, const StepArgs *da, const LaunchShape &ls, int k, hipStream_t s);
-template size_t resident_lds<4>(int th);
+template size_t resident_lds<4>(int L, int rows);
 template hipError_t resident_n<4>(int L, const ResidentArgs &r, const ResidentPlan &p, hipStream_t s);
 
 }  // namespace ifos

@@ -15,8 +15,8 @@
 // out of its registers and its path; with more rows the instructions issued.
 // The per-step kernels pay two launches a step, each with its ramp, drain and
 // cold loads.  Time per forward step, those and this (us): FDORDER 8, L=2:
-// 1024x256 13.2 / 5.6, 1024x512 20.0 / 13.0, 1024x768 26.5 / 21.4; elastic:
-// 1200x600 FDORDER 8 18.9 / 11.4, 1024x256 FDORDER 4 10.2 / 5.1.
+// 1024x256 13.2 / 5.6, 1024x512 20.2 / 10.6, 1024x768 26.4 / 17.5; elastic:
+// 1200x600 FDORDER 8 18.9 / 11.2, 1024x256 FDORDER 4 10.2 / 5.1.
 #pragma once
 #include "ifos_step.h"
 
@@ -24,13 +24,25 @@ namespace ifos {
 
 constexpr int kResidentThreads = 1024;  // largest workgroup: 64 columns x 16 rows of threads
 
-// Rows of cells per thread the kernel is compiled for, by the number of
-// relaxation mechanisms (0: not compiled).  1024 threads share a compute unit's
-// registers, 128 each; with these counts at most a few dozen values spill and
-// the run is faster than the per-step kernels' (us per forward step of a full
-// chip, FDORDER 8: elastic, four rows 25.1 / 17.3, L=2, three rows 26.5 / 21.4,
-// L=3, two rows 22.0 / 16.4).
-constexpr int resident_max_rows(int L) { return L == 0 ? 4 : L <= 2 ? 3 : L <= 3 ? 2 : 0; }
+// Rows of cells per thread the kernel is compiled for, by the stencil reach and
+// the number of relaxation mechanisms (0: not compiled).  1024 threads share a
+// compute unit's registers, 128 each, and its LDS.  us per forward step of a full
+// chip, per-step kernels and this, FDORDER 8: elastic, four rows 25.9 / 15.5, six
+// 33.6 / 29.4; L=1, four 28.8 / 25.0; L=2, three 26.4 / 17.9, four 31.1 / 27.7;
+// L=3, three 28.1 / 25.5.  Four rows with L=2 spill too much beyond FDORDER 8
+// (FDORDER 12: 35.0 / 34.7, a gradient 77.1 / 78.3).
+constexpr int resident_max_rows(int N, int L) { return L == 0 ? 6 : L == 1 || (L == 2 && N <= 4) ? 4 : L <= 3 ? 3 : 0; }
+
+// Where the registers spill most the tiles have to be nearly full: a tile just
+// over the height of one row fewer takes as long as a full one.  Elastic,
+// FDORDER 8, a gradient's pair of steps (us): 65 rows of cells 55.9 / 57.5, 72
+// 60.5 / 54.7; L=2, 49 rows 59.5 / 62.3, 56 64.3 / 61.3; L=3, 33 rows 48.6 / 49.8,
+// 40 55.4 / 53.2.
+constexpr bool resident_pays(int N, int L, int rows, int th)
+{
+    const bool crowded = N >= 4 && rows >= (L == 0 ? 5 : L == 3 ? 3 : 4) && L != 1;
+    return !crowded || th >= 16 * rows - 8;
+}
 
 constexpr int kWordsPerThread = 3;  // inbox words a thread polls, one row per thread
 

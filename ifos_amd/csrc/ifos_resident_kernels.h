@@ -9,25 +9,39 @@
 
 namespace ifos {
 
-// Offsets of the LDS arrays of a tile, in floats.  Row r, column x of the
-// tile (0-based) sit at vx, vy, sxy: (r + N) * W + x + N; sxx (no rows above
-// and below): r * W + x + N; syy (no columns to the sides): (r + N) * 64 + x.
-template <int N>
+// Offsets of the LDS arrays of a tile, in floats, for the highest tile of R rows
+// per thread (compile-time, so that one address register serves several arrays
+// through the instructions' offsets).  Row r, column x of the tile (0-based) sit
+// at vx, vy, sxy: (r + N) * W + x + N; sxx (no rows above and below): r * W + x +
+// N; syy (no columns to the sides): (r + N) * 64 + x.
+template <int N, int R>
 struct ResLds {
-    static constexpr int W = kTileX + 2 * N;
-    __host__ __device__ static int vx(int) { return 0; }
-    __host__ __device__ static int vy(int th) { return (th + 2 * N) * W; }
-    __host__ __device__ static int sxy(int th) { return 2 * (th + 2 * N) * W; }
-    __host__ __device__ static int sxx(int th) { return 3 * (th + 2 * N) * W; }
-    __host__ __device__ static int syy(int th) { return 3 * (th + 2 * N) * W + th * W; }
-    __host__ __device__ static int maxima(int th) { return syy(th) + (th + 2 * N) * kTileX; }
+    static constexpr int W = kTileX + 2 * N, TH = kResidentThreads / kTileX * R, H = TH + 2 * N;
+    static constexpr int vx = 0, vy = H * W, sxy = 2 * H * W, sxx = 3 * H * W, syy = 3 * H * W + TH * W;
+    static constexpr int maxima = syy + H * kTileX;  // of 16-bit snapshots, 5 per row
     // CPML profiles of the columns (6 floats, then 2 doubles, [.][64]) and of
     // the rows ([row] of 6 floats and 2 doubles), moduli of the surface row
-    __host__ __device__ static int xprof(int th) { return (maxima(th) + 5 * th + 1) / 2 * 2; }
-    __host__ __device__ static int yprof(int th) { return xprof(th) + 10 * kTileX; }
-    __host__ __device__ static int surface(int th) { return yprof(th) + 10 * th; }
-    __host__ __device__ static int total(int th) { return surface(th) + 4 * kTileX; }
+    static constexpr int xprof = (maxima + 5 * TH + 1) / 2 * 2, yprof = xprof + 10 * kTileX;
+    static constexpr int surface = yprof + 10 * TH;
+    static constexpr int planes = surface + 4 * kTileX;  // per-cell coefficients outside registers, [plane][row][64]
+    static constexpr int plane = TH * kTileX;
 };
+
+// Coefficients of a cell: 2 d, e, dip per mechanism, 2 f, g, fipjp (the latter
+// three alone when elastic), DT times the two buoyancies.
+constexpr int coefficients(int L) { return 3 * L + 5; }
+
+// How many of them, the first in that order, sit in LDS instead of registers:
+// none with one row per thread, else as many as fit beside the largest tile.
+// (With all of them in registers 36 values of every thread spilled to scratch on
+// 1024x512, L=2, FDORDER 8, and a step took 13.0 us instead of 10.6.)
+template <int N, int L, int R>
+constexpr int lds_coefficients()
+{
+    if (R == 1) return 0;
+    const int n = ((163840 - 256) / 4 - ResLds<N, R>::planes) / ResLds<N, R>::plane;
+    return n < 0 ? 0 : n < coefficients(L) ? n : coefficients(L);
+}
 
 // The argument block, read afresh: what a block of code needs of it is loaded
 // there (scalar loads that hit the constant cache) instead of staying in
@@ -262,7 +276,7 @@ __device__ __forceinline__ float res_snap_load(A &a, int s, int f, long k, unsig
 template <int N, int L, int R>
 __global__ __launch_bounds__(kResidentThreads) void k_resident(const ResidentArgs ra)
 {
-    using D = ResLds<N>;
+    using D = ResLds<N, R>;
     constexpr int W = D::W, M = 2 * N - 1, L1 = L > 0 ? L : 1;
     const ArgPtr pa = cmem(ra.a);
     const auto &a = *pa;
@@ -280,14 +294,14 @@ __global__ __launch_bounds__(kResidentThreads) void k_resident(const ResidentArg
 #pragma unroll
     for (int r = 0; r < R; r++) live[r] = i <= NX && j + r <= NY;
 
-    // ---- LDS, all zero (fields, and what lies outside the grid for good)
-    for (int q = ty * kTileX + tx; q < D::total(th); q += kTileX * ra.ty) lds[q] = 0.0f;
+    // ---- the fields in LDS, all zero (what lies outside the grid stays so)
+    for (int q = ty * kTileX + tx; q < D::maxima; q += kTileX * ra.ty) lds[q] = 0.0f;
     if (tx == 0 && ty == 0) s_stop = 0;
     // offsets of row 0, column 0
-    const int oVX = D::vx(th) + N * W + N, oVY = D::vy(th) + N * W + N, oSXY = D::sxy(th) + N * W + N;
-    const int oSXX = D::sxx(th) + N, oSYY = D::syy(th) + N * kTileX;
+    constexpr int oVX = D::vx + N * W + N, oVY = D::vy + N * W + N, oSXY = D::sxy + N * W + N;
+    constexpr int oSXX = D::sxx + N, oSYY = D::syy + N * kTileX;
     float *const VX = lds + oVX, *const VY = lds + oVY, *const SXY = lds + oSXY, *const SXX = lds + oSXX;
-    float *const SYY = lds + oSYY, *const maxima = lds + D::maxima(th);
+    float *const SYY = lds + oSYY, *const maxima = lds + D::maxima;
 
     // ---- neighbours
     const int sides = (by + 1 < ra.tiles_y ? kBelow : 0) | (by > 0 ? kAbove : 0) | (bx + 1 < a.nbx ? kRight : 0) |
@@ -331,9 +345,19 @@ __global__ __launch_bounds__(kResidentThreads) void k_resident(const ResidentArg
     // buoyancies stay beside their products with DT; else they are read again
     // where they are needed (snapshots, point forces).
     constexpr bool kOne = R == 1;
-    float ripk = 0.0f, rjpk = 0.0f, dtx[R], dty[R];
-    float f2[R], gl[R], fip[R];                  // elastic: 2 f, g, fipjp
-    ViscUpdate<L1> vu[R];
+    float ripk = 0.0f, rjpk = 0.0f;
+    constexpr int NC = coefficients(L), NP = lds_coefficients<N, L, R>(), NR = NC > NP ? NC - NP : 1;
+    constexpr int cF2 = 3 * L, cG = 3 * L + 1, cFip = 3 * L + 2, cDtx = 3 * L + 3, cDty = 3 * L + 4;
+    float creg[R][NR];
+    float *const clds = lds + D::planes + r0 * kTileX + tx;
+    auto coef = [&](int r, int k) -> float {
+        if (k < NP) return clds[k * D::plane + r * kTileX];
+        return creg[r][k - NP];
+    };
+    auto set_coef = [&](int r, int k, float v) {
+        if (k < NP) clds[k * D::plane + r * kTileX] = v;
+        else creg[r][k - NP] = v;
+    };
     float rr[R][L1], pp[R][L1], qq[R][L1];
     float eta[L1 + 1], bip[L1 + 1], bjm[L1 + 1], cip[L1 + 1], cjm[L1 + 1], hc[N + 1];
 #pragma unroll
@@ -351,19 +375,29 @@ __global__ __launch_bounds__(kResidentThreads) void k_resident(const ResidentArg
         const unsigned ci = (live[r] ? c + r * P : P + 1u) * 4u;  // cell (1, 1): every grid has it
         const float bx_ = at(gmem(a.rip), ci), by_ = at(gmem(a.rjp), ci);
         if (r == 0) ripk = bx_, rjpk = by_;
-        dtx[r] = g.DT * bx_;
-        dty[r] = g.DT * by_;
+        set_coef(r, cDtx, g.DT * bx_);
+        set_coef(r, cDty, g.DT * by_);
         if (L == 0) {
-            f2[r] = 2.0f * at(gmem(a.f), ci);
-            gl[r] = at(gmem(a.gl), ci);
-            fip[r] = at(gmem(a.uipjp), ci);
+            set_coef(r, cF2, 2.0f * at(gmem(a.f), ci));
+            set_coef(r, cG, at(gmem(a.gl), ci));
+            set_coef(r, cFip, at(gmem(a.uipjp), ci));
         } else {
             ViscCell vc;
             visc_coeffs(L, g.DT, at(gmem(a.mu), ci), at(gmem(a.pi), ci), at(gmem(a.muipjp), ci),
                         at(gmem(a.taus), ci), at(gmem(a.taup), ci), at(gmem(a.tausipjp), ci), vc);
-            visc_update(vc, eta, vu[r]);
+            ViscUpdate<L1> v;
+            visc_update(vc, eta, v);
+#pragma unroll
+            for (int l = 0; l < L; l++) {
+                set_coef(r, 3 * l, v.d2[l]);
+                set_coef(r, 3 * l + 1, v.e[l]);
+                set_coef(r, 3 * l + 2, v.dip[l]);
+            }
+            set_coef(r, cF2, v.f2);
+            set_coef(r, cG, v.g);
+            set_coef(r, cFip, v.fipjp);
             if (r == 0 && ty == 0) {
-                float *const sf = lds + D::surface(th) + tx;
+                float *const sf = lds + D::surface + tx;
                 sf[0] = vc.mu;
                 sf[kTileX] = vc.pi;
                 sf[2 * kTileX] = vc.taus;
@@ -410,12 +444,12 @@ __global__ __launch_bounds__(kResidentThreads) void k_resident(const ResidentArg
     if (inx) xp = profile(hx, g.pml.K_x, g.pml.a_x, g.pml.b_x, g.pml.K_xh, g.pml.a_xh, g.pml.b_xh);
     if (kOne && strip(j, NY, !fs) >= 0)
         yp = profile(strip(j, NY, !fs), g.pml.K_y, g.pml.a_y, g.pml.b_y, g.pml.K_yh, g.pml.a_yh, g.pml.b_yh);
-    float *const xl = lds + D::xprof(th) + tx, *const yl = lds + D::yprof(th);
+    float *const xl = lds + D::xprof + tx, *const yl = lds + D::yprof;
     if (!kOne) {
         if (ty == 0) {
             xl[0] = xp.K; xl[kTileX] = xp.a; xl[2 * kTileX] = xp.b;
             xl[3 * kTileX] = xp.Kh; xl[4 * kTileX] = xp.ah; xl[5 * kTileX] = xp.bh;
-            double *const xd2 = (double *)(lds + D::xprof(th) + 6 * kTileX) + tx;
+            double *const xd2 = (double *)(lds + D::xprof + 6 * kTileX) + tx;
             xd2[0] = xp.rK;
             xd2[kTileX] = xp.rKh;
         }
@@ -431,7 +465,7 @@ __global__ __launch_bounds__(kResidentThreads) void k_resident(const ResidentArg
     }
     auto column = [&]() {
         if constexpr (kOne) return xp;
-        const double *const xd2 = (const double *)(lds + D::xprof(th) + 6 * kTileX) + tx;
+        const double *const xd2 = (const double *)(lds + D::xprof + 6 * kTileX) + tx;
         return Profile{xl[0], xl[kTileX], xl[2 * kTileX], xl[3 * kTileX], xl[4 * kTileX], xl[5 * kTileX], xd2[0],
                        xd2[kTileX]};
     };
@@ -561,7 +595,7 @@ __global__ __launch_bounds__(kResidentThreads) void k_resident(const ResidentArg
                     at(gmem(bv.psi_sxy_y) + po, ky) = q4;
                 }
                 const float sumx = sxx_x + sxy_y, sumy = sxy_x + syy_y;
-                float vx = dtx[r] * sumx, vy = dty[r] * sumy;  // vel_new
+                float vx = coef(r, cDtx) * sumx, vy = coef(r, cDty) * sumy;  // vel_new
                 div_by2(vx, vy, DH, DH, rDH, rDH);
                 vx = vx0 + vx;
                 vy = vy0 + vy;
@@ -688,15 +722,25 @@ __global__ __launch_bounds__(kResidentThreads) void k_resident(const ResidentArg
                 }
                 float ux = 0.0f, uy = 0.0f, uxy = 0.0f;
                 if (L == 0) {
+                    const float f2 = coef(r, cF2), gl = coef(r, cG), fip = coef(r, cFip);
                     if (rates)
-                        rates_elastic(0.5f * afresh(f2[r]), afresh(gl[r]), afresh(fip[r]), afresh(DT), vxx, vyx, vxy,
-                                      vyy, ux, uy, uxy);
-                    stress_elastic(f2[r], gl[r], fip[r], vxx, vyx, vxy, vyy, sxx, syy, sxy);
+                        rates_elastic(0.5f * afresh(f2), afresh(gl), afresh(fip), afresh(DT), vxx, vyx, vxy, vyy, ux,
+                                      uy, uxy);
+                    stress_elastic(f2, gl, fip, vxx, vyx, vxy, vyy, sxx, syy, sxy);
                 } else {
-                    ViscUpdate<L1> v = vu[r];
+                    ViscUpdate<L1> v;
+                    v.f2 = coef(r, cF2);
+                    v.g = coef(r, cG);
+                    v.fipjp = coef(r, cFip);
                     if (!kOne) v.f2 = afresh(v.f2);  // its FP64 value need not stay in registers
-                    stress_visc(v, bip, bjm, cip, cjm, dthalbe, afresh(DT), vxx, vyx, vxy, vyy, sxx, syy, sxy, rr[r], pp[r], qq[r],
-                                rates, ux, uy, uxy);
+#pragma unroll
+                    for (int l = 0; l < L; l++) {
+                        v.d2[l] = coef(r, 3 * l);
+                        v.e[l] = coef(r, 3 * l + 1);
+                        v.dip[l] = coef(r, 3 * l + 2);
+                    }
+                    stress_visc(v, bip, bjm, cip, cjm, dthalbe, afresh(DT), vxx, vyx, vxy, vyy, sxx, syy, sxy, rr[r],
+                                pp[r], qq[r], rates, ux, uy, uxy);
                 }
                 if (explosive && (inj_rows >> r & 1u)) {
                     const auto &b = *afresh(pa);
@@ -743,9 +787,9 @@ __global__ __launch_bounds__(kResidentThreads) void k_resident(const ResidentArg
                             *ps = v;
                         }
                         if (L == 0) {
-                            surface_elastic_update(afresh(f2[r]), afresh(gl[r]), DT, dx, dy, sxx, rates, ux);
+                            surface_elastic_update(afresh(coef(r, cF2)), afresh(coef(r, cG)), DT, dx, dy, sxx, rates, ux);
                         } else {
-                            const float *const sf = lds + D::surface(th) + tx;
+                            const float *const sf = lds + D::surface + tx;
                             surface_visc_update<L1>(sf[0], sf[kTileX], sf[2 * kTileX], sf[3 * kTileX], eta, DT, dx,
                                                     dy, sxx, pp[r], rates, ux);
                         }
@@ -827,11 +871,26 @@ __global__ __launch_bounds__(kResidentThreads) void k_resident(const ResidentArg
         }
 }
 
-// LDS bytes of a tile (host)
-template <int N>
-size_t resident_lds(int th)
+// LDS bytes of a workgroup (host)
+template <int N, int L, int R>
+static size_t resident_lds_rows(int rows)
 {
-    return sizeof(float) * (size_t)ResLds<N>::total(th);
+    typedef ResLds<N, R> D;
+    if (rows == R) return sizeof(float) * (size_t)(D::planes + lds_coefficients<N, L, R>() * D::plane);
+    if constexpr (R < resident_max_rows(N, L)) return resident_lds_rows<N, L, R + 1>(rows);
+    return (size_t)-1;
+}
+
+template <int N>
+size_t resident_lds(int L, int rows)
+{
+    switch (L) {
+    case 0: return resident_lds_rows<N, 0, 1>(rows);
+    case 1: return resident_lds_rows<N, 1, 1>(rows);
+    case 2: return resident_lds_rows<N, 2, 1>(rows);
+    case 3: return resident_lds_rows<N, 3, 1>(rows);
+    default: return (size_t)-1;
+    }
 }
 
 template <int N, int L, int R>
@@ -848,7 +907,7 @@ template <int N, int L, int R = 1>
 static hipError_t resident_rows(const ResidentArgs &r, const ResidentPlan &p, hipStream_t s)
 {
     if (p.rows == R) return resident_launch<N, L, R>(r, p, s);
-    if constexpr (R < resident_max_rows(L)) return resident_rows<N, L, R + 1>(r, p, s);
+    if constexpr (R < resident_max_rows(N, L)) return resident_rows<N, L, R + 1>(r, p, s);
     return hipErrorInvalidValue;
 }
 

@@ -16,7 +16,7 @@ void str_n(const StepArgs &a, const StepArgs *da, const LaunchShape &ls, int k, 
 template <int N>
 void fused_n(const StepArgs &a, const StepArgs *da, const LaunchShape &ls, int k, hipStream_t s);
 template <int N>
-size_t resident_lds(int th);
+size_t resident_lds(int L, int rows);
 template <int N>
 hipError_t resident_n(int L, const ResidentArgs &r, const ResidentPlan &p, hipStream_t s);
 
@@ -116,15 +116,15 @@ void launch_fused_step(const StepArgs &a, const StepArgs *da, const LaunchShape 
     }
 }
 
-static size_t lds_of(int N, int th)
+static size_t lds_of(int N, int L, int rows)
 {
     switch (N) {
-    case 1: return resident_lds<1>(th);
-    case 2: return resident_lds<2>(th);
-    case 3: return resident_lds<3>(th);
-    case 4: return resident_lds<4>(th);
-    case 5: return resident_lds<5>(th);
-    default: return resident_lds<6>(th);
+    case 1: return resident_lds<1>(L, rows);
+    case 2: return resident_lds<2>(L, rows);
+    case 3: return resident_lds<3>(L, rows);
+    case 4: return resident_lds<4>(L, rows);
+    case 5: return resident_lds<5>(L, rows);
+    default: return resident_lds<6>(L, rows);
     }
 }
 
@@ -135,7 +135,7 @@ static size_t lds_of(int N, int th)
 ResidentPlan resident_plan(const StepGeom &g, int L, int nslots, int snap_prec, int ncu, size_t lds_max)
 {
     ResidentPlan p;
-    const int most = resident_max_rows(L), nbx = (g.NX + kTileX - 1) / kTileX;
+    const int most = resident_max_rows(g.N, L), nbx = (g.NX + kTileX - 1) / kTileX;
     // periodic sides wrap the halo, which may span two tiles there
     if (g.BOUNDARY || most == 0 || nslots < 1 || (long)nbx * nslots > ncu) return p;
     const int across = ncu / (nbx * nslots);  // tile rows per slot that fit
@@ -152,8 +152,8 @@ ResidentPlan resident_plan(const StepGeom &g, int L, int nslots, int snap_prec, 
         p.tiles_y = (g.NY + p.th - 1) / p.th;
         p.nwg = nbx * p.tiles_y * nslots;
         p.words = (2 * g.N - 1) * 2 * (kTileX + p.th);
-        p.lds = lds_of(g.N, p.th);
-        if (p.lds + 64 <= lds_max) p.rows = rows;
+        p.lds = lds_of(g.N, L, rows);
+        if (p.lds + 64 <= lds_max && resident_pays(g.N, L, rows, th)) p.rows = rows;
         return p;
     }
     return p;

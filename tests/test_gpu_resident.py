@@ -54,17 +54,22 @@ def test_resident_equals_per_step_kernels(gpu_lib, c, kw):
     assert used and same_bits(want, have)
 
 
-@pytest.mark.parametrize("c", [dict(NX=64, NY=4096, L=0), dict(NX=64, NY=4097, L=2), dict(NX=1024, NY=256, L=1),
-                               dict(NX=1024, NY=257, L=0), dict(NX=900, NY=530, L=0), dict(NX=900, NY=700, L=2), dict(NX=960, NY=1024, L=0)],
-                         ids=lambda c: f"{c['NX']}x{c['NY']}_L{c['L']}")
-@pytest.mark.parametrize("order", [2, 8])
-def test_resident_large_tiles(gpu_lib, c, order):
+# NX, NY, L: the lowest and highest tiles of the row counts on 256 compute units,
+# and the highest order for which the run takes them
+LARGE = [(64, 4096, 0, 12), (64, 4097, 2, 12), (1024, 512, 1, 12), (1024, 640, 3, 12), (960, 816, 2, 12),
+         (1024, 768, 3, 12), (1024, 896, 2, 8), (1024, 1024, 1, 12), (900, 1224, 0, 12), (1024, 1408, 0, 8),
+         (1024, 1536, 0, 8), (1024, 513, 3, 2)]
+
+
+@pytest.mark.parametrize("NX,NY,L,highest", LARGE)
+@pytest.mark.parametrize("order", [2, 8, 12])
+def test_resident_large_tiles(gpu_lib, NX, NY, L, highest, order):
     """Every row count, from one row per thread of a full chip to the largest tile."""
-    w = workloads.small_case(seed=8, NT=12, FW=10, DTINV=2, VELOCITY=1, FDORDER=order, **c)
-    print(f"[resident] {c} FDORDER {order}", flush=True)
+    w = workloads.small_case(seed=8, NX=NX, NY=NY, L=L, NT=12, FW=10, DTINV=2, VELOCITY=1, FDORDER=order)
+    print(f"[resident] {NX}x{NY} L={L} FDORDER {order}", flush=True)
     want, _ = outputs(w, 0)
     have, used = outputs(w, 1)
-    assert used and same_bits(want, have)
+    assert same_bits(want, have) and used == (order <= highest)
 
 
 def test_run_given_up_is_repeated(gpu_lib):
