@@ -129,7 +129,6 @@ __device__ __forceinline__ void vel_rows_with(const StepArgs &a, int s, int blk,
                 cpml_velocity(g, j + r, i, a.psi_sxx_x + po, a.psi_sxy_x + po, a.psi_syy_y + po, a.psi_sxy_y + po,
                               sxx_x[r], sxy_x[r], sxy_y[r], syy_y[r]);
     }
-    const bool points = tile_has(a.inj, s, a.nbx * a.nby, blk);
     if (flags & kForward) {
         if (flags & kSnapStep) {
             float val[R][2];
@@ -163,7 +162,7 @@ __device__ __forceinline__ void vel_rows_with(const StepArgs &a, int s, int blk,
         vy[r] = vel_new(vy0[r], g.DT, rjp[r], sxy_x[r] + syy_y[r], g.DH);
     }
     // point forces / residual injection of these cells, in order
-    if (points) {
+    if (tile_has(a.inj, s, a.nbx * a.nby, blk)) {
 #pragma unroll
         for (int r = 0; r < R; r++)
             if (live[r])
@@ -394,15 +393,6 @@ __device__ __forceinline__ void str_cell(const StepArgs &a, int s, int blk, int 
     const bool snap_step = (flags & kSnapStep) != 0;
     const bool corr_step = (flags & kCorrStep) != 0;
     const bool rates = snap_step && a.VELOCITY == 1;
-    // the explosive sources and receivers of this cell, looked up before the
-    // stencil work so that the latency is hidden behind it
-    int ex = -1, rc = -1;
-    if ((flags & kForward) && live) {
-        const int nt_ = a.nbx * a.nby;
-        ex = first_point(a, a.exp, s, e, cmem(a.explosive)[s] && tile_has(a.exp, s, nt_, blk));
-        rc = first_point(a, a.rec, s, e, tile_has(a.rec, s, nt_, blk));
-    }
-
     float sxx = 0.0f, syy = 0.0f, sxy = 0.0f, ux = 0.0f, uy = 0.0f, uxy = 0.0f;
     float rr[L > 0 ? L : 1], pp[L > 0 ? L : 1], qq[L > 0 ? L : 1];
     if (live) {
@@ -430,10 +420,16 @@ __device__ __forceinline__ void str_cell(const StepArgs &a, int s, int blk, int 
         }
         // explosive sources of this cell, applied after the stress update
         // and before the free surface (src/IFOS2D.c:1758-1773)
-        for (int l = ex; l >= 0; l = gmem(a.exp.next)[l]) {
-            const float amp = explosive_amp(a.exp.sig + (long)l * a.NT - 1, nt, a.NT, g.DH);
-            sxx = add_half(sxx, amp);
-            syy = add_half(syy, amp);
+        // the look-ups of points come last: a tile without any (nearly all) would
+        // wait for their scalar loads before it issued its stencil loads (stress
+        // step of 2000x800, L=2: 27.6 us with them first, 26.4 so)
+        if (flags & kForward) {
+            const int ex = first_point(a, a.exp, s, e, tile_has(a.exp, s, a.nbx * a.nby, blk) && cmem(a.explosive)[s]);
+            for (int l = ex; l >= 0; l = gmem(a.exp.next)[l]) {
+                const float amp = explosive_amp(a.exp.sig + (long)l * a.NT - 1, nt, a.NT, g.DH);
+                sxx = add_half(sxx, amp);
+                syy = add_half(syy, amp);
+            }
         }
     }
     if (top) {
@@ -493,9 +489,12 @@ __device__ __forceinline__ void str_cell(const StepArgs &a, int s, int blk, int 
         gmem(a.wc)[wco + e] = w;
         gmem(a.wc_u)[wco + e] = wu;
     }
-    for (int t = rc; t >= 0; t = gmem(a.rec.next)[t]) {
-        gmem(a.seis_vx)[(long)t * a.NT + nt - 1] = vxs[c];
-        gmem(a.seis_vy)[(long)t * a.NT + nt - 1] = vys[c];
+    if (flags & kForward) {
+        const int rc = first_point(a, a.rec, s, e, tile_has(a.rec, s, a.nbx * a.nby, blk));
+        for (int t = rc; t >= 0; t = gmem(a.rec.next)[t]) {
+            gmem(a.seis_vx)[(long)t * a.NT + nt - 1] = vxs[c];
+            gmem(a.seis_vy)[(long)t * a.NT + nt - 1] = vys[c];
+        }
     }
     if (a.nan_flag && j == g.NY / 2 && i == g.NX / 2) {
         const float v = vys[c];
