@@ -222,6 +222,32 @@ static float *pad_copy(const float *src, int NX, int NY)
     return a;
 }
 
+void ifos_setup_relaxation(const ifos_config *c, ifos_materials *m)
+{
+    const int L = c->L;
+    if (!L) return;
+    /* eta (src/readmod.c:47-51) and prepare_update_s (src/prepare_update_s.c:21-108) */
+    float pts[IFOS_MAXL + 1];
+    for (int l = 1; l <= L; l++) {
+        pts[l] = 1.0 / (2.0 * IFOS_PI * c->FL[l]);
+        m->eta[l] = c->DT / pts[l];
+    }
+    float ws = 2.0 * IFOS_PI * c->F_REF;
+    float sumu = 0.0, sumpi = 0.0;
+    for (int l = 1; l <= L; l++) {
+        sumu = sumu + ((ws * ws * pts[l] * pts[l]) / (1.0 + ws * ws * pts[l] * pts[l]));
+        sumpi = sumpi + ((ws * ws * pts[l] * pts[l]) / (1.0 + ws * ws * pts[l] * pts[l]));
+    }
+    m->sumu = sumu;
+    m->sumpi = sumpi;
+    for (int l = 1; l <= L; l++) {
+        m->bip[l] = 1.0 / (1.0 + (m->eta[l] * 0.5));
+        m->bjm[l] = 1.0 / (1.0 + (m->eta[l] * 0.5));
+        m->cip[l] = 1.0 - (m->eta[l] * 0.5);
+        m->cjm[l] = 1.0 - (m->eta[l] * 0.5);
+    }
+}
+
 int ifos_setup_materials(const ifos_config *c, const float *vp, const float *vs, const float *rho,
                          const float *taus, const float *taup, ifos_materials *m)
 {
@@ -261,26 +287,8 @@ int ifos_setup_materials(const ifos_config *c, const float *vp, const float *vs,
             m->g[k] = rr * ((pp * pp) - 2 * uu * uu);
         }
     if (L) {
-        /* eta (src/readmod.c:47-51) and prepare_update_s (src/prepare_update_s.c:21-108) */
-        float pts[IFOS_MAXL + 1];
-        for (int l = 1; l <= L; l++) {
-            pts[l] = 1.0 / (2.0 * IFOS_PI * c->FL[l]);
-            m->eta[l] = c->DT / pts[l];
-        }
-        float ws = 2.0 * IFOS_PI * c->F_REF;
-        float sumu = 0.0, sumpi = 0.0;
-        for (int l = 1; l <= L; l++) {
-            sumu = sumu + ((ws * ws * pts[l] * pts[l]) / (1.0 + ws * ws * pts[l] * pts[l]));
-            sumpi = sumpi + ((ws * ws * pts[l] * pts[l]) / (1.0 + ws * ws * pts[l] * pts[l]));
-        }
-        m->sumu = sumu;
-        m->sumpi = sumpi;
-        for (int l = 1; l <= L; l++) {
-            m->bip[l] = 1.0 / (1.0 + (m->eta[l] * 0.5));
-            m->bjm[l] = 1.0 / (1.0 + (m->eta[l] * 0.5));
-            m->cip[l] = 1.0 - (m->eta[l] * 0.5);
-            m->cjm[l] = 1.0 - (m->eta[l] * 0.5);
-        }
+        ifos_setup_relaxation(c, m);
+        const float sumu = m->sumu, sumpi = m->sumpi;
         m->fipjp = (float *)malloc(n * sizeof(float));
         m->d = (float *)malloc(n * L * sizeof(float));
         m->e = (float *)malloc(n * L * sizeof(float));

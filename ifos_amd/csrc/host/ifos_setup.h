@@ -28,6 +28,9 @@ typedef struct ifos_materials {
 
 int ifos_setup_materials(const ifos_config *c, const float *vp, const float *vs, const float *rho,
                          const float *taus, const float *taup, ifos_materials *m);
+/* the scalars of the relaxation mechanisms (eta, bip, bjm, cip, cjm, sumu,
+ * sumpi) alone; nothing with L = 0 */
+void ifos_setup_relaxation(const ifos_config *c, ifos_materials *m);
 void ifos_free_materials(ifos_materials *m);
 
 /* Butterworth low- or highpass of the given order and corner fc (Hz) for

@@ -101,6 +101,10 @@ static hipError_t dfree(void *p)
 // up and repeated with the per-step kernels.
 constexpr unsigned long long kResidentLimit = 20000000ull;
 
+// padded material grids, and [NY][NX] planes shared by the shots
+constexpr int kMaterialGrids = 11;
+constexpr int interior_planes(int L) { return L ? 13 : 11; }
+
 struct ifos_engine {
     ifos_config c;
     int device = 0;
@@ -124,13 +128,13 @@ struct ifos_engine {
     int last_set = 0;     // wavefield set holding the state after the last run
     // shared material grids
     float *mslab = nullptr;
-    float *rip, *rjp, *uipjp, *f, *g, *fipjp, *rho, *vs, *vp, *taus, *taup;
-    float *d = nullptr, *e = nullptr, *dip = nullptr;
+    float *rip, *rjp, *uipjp, *f, *g, *taus, *taup;
     float *mu_r, *pi_r, *muipjp_r, *tausipjp;  // relaxed moduli for the in-kernel GSLS coefficients
 
     // interior [NY][NX]
     float *interior = nullptr;
     float *muss, *lamss, *vs_i, *vp_i, *rho_i, *g_vp, *g_vs, *g_rho, *s_vp, *s_vs, *s_rho;
+    float *taus_i = nullptr, *taup_i = nullptr;  // L > 0
     float *wcbuf = nullptr;  // per slot: wc, wc_u, wc_rho (3 planes)
 
     // CPML
@@ -318,33 +322,27 @@ static int engine_create(const ifos_config *cfg, int device, int slots, ifos_eng
         E->q = next(); for (int l = 1; l < L; l++) next();
     }
     E->vx2 = next(); E->vy2 = next(); E->sxx2 = next(); E->syy2 = next(); E->sxy2 = next();
-    // shared: 15 material grids + 3L coefficient planes
-    const int nmat = 15 + 3 * L;
+    // shared: material grids
+    const int nmat = kMaterialGrids;
     if (dmalloc(&E->mslab, sizeof(float) * E->field * nmat) != hipSuccess) {
         ifos_set_error("device allocation of %d material grids failed", nmat);
         return fail(-3);
     }
     hipMemsetAsync(E->mslab, 0, sizeof(float) * E->field * nmat, E->stream);
     gp = E->mslab + E->off;
-    E->rip = next(); E->rjp = next(); E->uipjp = next(); E->f = next(); E->g = next(); E->fipjp = next();
-    E->rho = next(); E->vs = next(); E->vp = next(); E->taus = next(); E->taup = next();
+    E->rip = next(); E->rjp = next(); E->uipjp = next(); E->f = next(); E->g = next();
+    E->taus = next(); E->taup = next();
     E->mu_r = next(); E->pi_r = next(); E->muipjp_r = next(); E->tausipjp = next();
-    if (L) {
-        E->d = next(); for (int l = 1; l < L; l++) next();
-        E->e = next(); for (int l = 1; l < L; l++) next();
-        E->dip = next(); for (int l = 1; l < L; l++) next();
-    }
-
-    // interior arrays: 11 shared + 3 correlation planes per slot
-    const int nint = 11;
+    // interior arrays: shared, and 3 correlation planes per slot
+    const int nint = interior_planes(L);
     if (dmalloc(&E->interior, sizeof(float) * E->plane * nint) != hipSuccess ||
         dmalloc(&E->wcbuf, sizeof(float) * E->plane * 3 * slots) != hipSuccess) {
         ifos_set_error("device allocation of interior arrays failed");
         return fail(-3);
     }
     hipMemsetAsync(E->interior, 0, sizeof(float) * E->plane * nint, E->stream);
-    float **ia[nint] = {&E->muss, &E->lamss, &E->vs_i, &E->vp_i, &E->rho_i, &E->g_vp, &E->g_vs, &E->g_rho,
-                        &E->s_vp, &E->s_vs, &E->s_rho};
+    float **ia[] = {&E->muss, &E->lamss, &E->vs_i, &E->vp_i, &E->rho_i, &E->g_vp, &E->g_vs, &E->g_rho,
+                    &E->s_vp, &E->s_vs, &E->s_rho, &E->taus_i, &E->taup_i};
     for (int k = 0; k < nint; k++) *ia[k] = E->interior + (long)k * E->plane;
 
     // CPML profiles and per-slot memory
@@ -426,12 +424,59 @@ extern "C" void ifos_engine_destroy(ifos_engine *E)
 }
 
 // copy an interior [NY][NX] host array into a padded device grid
-static int upload_grid(ifos_engine *E, float *dst_origin, const float *host)
+// Materials of a model, one thread per cell: what ifos_setup_materials forms on
+// the host, operand for operand (the same bits), from the uploaded grids.  The
+// neighbours past the last row and column are the first ones (the halo of a
+// single-rank run, src/matcopy_elastic.c:48-140).  On one host core, with a
+// pitched copy for every grid, this took 15.0 ms of the 19.7 ms of a step-length
+// trial on 400x200.
+struct MaterialArgs {
+    int NX, NY, pitch, L;
+    float sumu, sumpi;
+    const float *vp, *vs, *rho, *taus, *taup;             // [NY][NX]
+    float *muss, *lamss;                                  // [NY][NX]
+    float *rip, *rjp, *uipjp, *f, *g;                     // padded grids (origin pointers)
+    float *taus_p, *taup_p, *mu, *pi, *muipjp, *tausipjp;  // L > 0
+};
+
+__global__ __launch_bounds__(256) void k_materials(MaterialArgs a)
 {
-    float *dst = dst_origin + pad_index(E, 1, 1);
-    HIP_TRY(hipMemcpy2DAsync(dst, sizeof(float) * E->pitch, host, sizeof(float) * E->c.NX, sizeof(float) * E->c.NX,
-                             E->c.NY, hipMemcpyHostToDevice, E->stream));
-    return 0;
+    const int i = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y * 4 + threadIdx.y;
+    if (i >= a.NX || j >= a.NY) return;
+    const long row = (long)j * a.NX, below = j + 1 < a.NY ? row + a.NX : 0;
+    const int right = i + 1 < a.NX ? i + 1 : 0;
+    const long k = row + i, c = (long)(j + 1) * a.pitch + i + 1;
+    const auto R = gmem(a.rho), U = gmem(a.vs), V = gmem(a.vp);
+    const float r1 = R[k], r2 = R[row + right], r3 = R[below + i], r4 = R[below + right];
+    const float v1 = U[k], v2 = U[row + right], v3 = U[below + i], v4 = U[below + right], p1 = V[k];
+    // av_rho (src/av_rho.c:27-31)
+    gmem(a.rjp)[c] = (float)(1.0 / (0.5 * (double)(r1 + r3)));
+    gmem(a.rip)[c] = (float)(1.0 / (0.5 * (double)(r1 + r2)));
+    // av_mue, PARAMETERIZATION 1 (src/av_mue.c:45-62)
+    const float u1 = r1 * v1 * v1, u2 = r2 * v2 * v2, u3 = r3 * v3 * v3, u4 = r4 * v4 * v4;
+    float u = (float)(4.0 / ((1.0 / (double)u1) + (1.0 / (double)u2) + (1.0 / (double)u3) + (1.0 / (double)u4)));
+    if (u1 == 0.0f || u2 == 0.0f || u3 == 0.0f || u4 == 0.0f) u = 0.0f;
+    gmem(a.uipjp)[c] = u;
+    // moduli of the correlation and chain rule (src/IFOS2D.c:2395-2396)
+    gmem(a.muss)[k] = u1;
+    gmem(a.lamss)[k] = (float)((double)(r1 * p1 * p1) - 2.0 * (double)u1);
+    if (a.L == 0) {
+        // update_s_elastic_PML (src/update_s_elastic_PML.c:228-230)
+        gmem(a.f)[c] = u1;
+        gmem(a.g)[c] = r1 * ((p1 * p1) - 2.0f * v1 * v1);
+        return;
+    }
+    // av_tau (src/av_tau.c:25-27), relaxed moduli of prepare_update_s
+    // (src/prepare_update_s.c:21-65)
+    const auto T = gmem(a.taus);
+    const float ts = T[k], tp = gmem(a.taup)[k];
+    const float ti = (float)(0.25 * (double)(ts + T[row + right] + T[below + i] + T[below + right]));
+    gmem(a.taus_p)[c] = ts;
+    gmem(a.taup_p)[c] = tp;
+    gmem(a.tausipjp)[c] = ti;
+    gmem(a.mu)[c] = (float)((double)(v1 * v1 * r1) / (1.0 + (double)(a.sumu * ts)));
+    gmem(a.pi)[c] = (float)((double)(p1 * p1 * r1) / (1.0 + (double)(a.sumpi * tp)));
+    gmem(a.muipjp)[c] = (float)((double)u / (1.0 + (double)(a.sumu * ti)));
 }
 
 extern "C" int ifos_engine_set_model(ifos_engine *E, const float *vp, const float *vs, const float *rho,
@@ -442,37 +487,25 @@ extern "C" int ifos_engine_set_model(ifos_engine *E, const float *vp, const floa
     if (c.L && (!taus || !taup)) return ifos_set_error("viscoelastic model needs taus and taup"), -2;
     HIP_TRY(hipStreamSynchronize(E->stream));
     E->snap_valid = false;
-    ifos_free_materials(&E->mat);
-    ifos_setup_materials(&c, vp, vs, rho, taus, taup, &E->mat);
-    ifos_materials &m = E->mat;
-    ENG_TRY(upload_grid(E, E->rip, m.rip));
-    ENG_TRY(upload_grid(E, E->rjp, m.rjp));
-    ENG_TRY(upload_grid(E, E->uipjp, m.uipjp));
-    ENG_TRY(upload_grid(E, E->f, m.f));
-    ENG_TRY(upload_grid(E, E->g, m.g));
-    ENG_TRY(upload_grid(E, E->rho, rho));
-    ENG_TRY(upload_grid(E, E->vs, vs));
-    ENG_TRY(upload_grid(E, E->vp, vp));
-    if (c.L) {
-        ENG_TRY(upload_grid(E, E->fipjp, m.fipjp));
-        ENG_TRY(upload_grid(E, E->taus, taus));
-        ENG_TRY(upload_grid(E, E->taup, taup));
-        ENG_TRY(upload_grid(E, E->mu_r, m.mu_r));
-        ENG_TRY(upload_grid(E, E->pi_r, m.pi_r));
-        ENG_TRY(upload_grid(E, E->muipjp_r, m.muipjp_r));
-        ENG_TRY(upload_grid(E, E->tausipjp, m.tausipjp));
-        for (int l = 0; l < c.L; l++) {
-            ENG_TRY(upload_grid(E, E->d + l * E->field, m.d + (size_t)l * E->plane));
-            ENG_TRY(upload_grid(E, E->e + l * E->field, m.e + (size_t)l * E->plane));
-            ENG_TRY(upload_grid(E, E->dip + l * E->field, m.dip + (size_t)l * E->plane));
-        }
-    }
+    ifos_setup_relaxation(&c, &E->mat);
     const size_t pb = sizeof(float) * E->plane;
-    HIP_TRY(hipMemcpyAsync(E->muss, m.muss, pb, hipMemcpyHostToDevice, E->stream));
-    HIP_TRY(hipMemcpyAsync(E->lamss, m.lamss, pb, hipMemcpyHostToDevice, E->stream));
-    HIP_TRY(hipMemcpyAsync(E->vs_i, vs, pb, hipMemcpyHostToDevice, E->stream));
     HIP_TRY(hipMemcpyAsync(E->vp_i, vp, pb, hipMemcpyHostToDevice, E->stream));
+    HIP_TRY(hipMemcpyAsync(E->vs_i, vs, pb, hipMemcpyHostToDevice, E->stream));
     HIP_TRY(hipMemcpyAsync(E->rho_i, rho, pb, hipMemcpyHostToDevice, E->stream));
+    if (c.L) {
+        HIP_TRY(hipMemcpyAsync(E->taus_i, taus, pb, hipMemcpyHostToDevice, E->stream));
+        HIP_TRY(hipMemcpyAsync(E->taup_i, taup, pb, hipMemcpyHostToDevice, E->stream));
+    }
+    MaterialArgs a;
+    a.NX = c.NX; a.NY = c.NY; a.pitch = E->pitch; a.L = c.L;
+    a.sumu = E->mat.sumu; a.sumpi = E->mat.sumpi;
+    a.vp = E->vp_i; a.vs = E->vs_i; a.rho = E->rho_i; a.taus = E->taus_i; a.taup = E->taup_i;
+    a.muss = E->muss; a.lamss = E->lamss;
+    a.rip = E->rip; a.rjp = E->rjp; a.uipjp = E->uipjp; a.f = E->f; a.g = E->g;
+    a.taus_p = E->taus; a.taup_p = E->taup; a.mu = E->mu_r; a.pi = E->pi_r;
+    a.muipjp = E->muipjp_r; a.tausipjp = E->tausipjp;
+    hipLaunchKernelGGL(k_materials, dim3((c.NX + 63) / 64, (c.NY + 3) / 4), dim3(64, 4), 0, E->stream, a);
+    HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(E->stream));
     E->model_set = true;
     return 0;
@@ -1584,8 +1617,8 @@ extern "C" size_t ifos_engine_bytes(const ifos_config *c, int slots, int snap_pr
     const size_t plane = (size_t)c->NX * c->NY;
     const int fw2 = c->FW > 0 ? 2 * c->FW : 1;
     size_t b = sizeof(float) * field * (size_t)(15 + 3 * c->L) * slots;   // wavefields, both sets
-    b += sizeof(float) * field * (size_t)(15 + 3 * c->L);                 // materials
-    b += sizeof(float) * plane * (11 + 3 * (size_t)slots);                // interior + correlation
+    b += sizeof(float) * field * kMaterialGrids;                          // materials
+    b += sizeof(float) * plane * (interior_planes(c->L) + 3 * (size_t)slots);  // interior + correlation
     b += sizeof(float) * (size_t)(7 * c->NY * fw2 + 6 * fw2 * c->NX) * slots;  // CPML memory
     b += sizeof(int) * 2 * plane * slots;                                 // cells of sources and receivers
     b += sizeof(float) * (size_t)6 * ntr_total * c->NT;                   // seismograms etc.
