@@ -4,7 +4,8 @@
 // (slot-major [k][j][i]), seismograms, adjoint sources and the gradient
 // accumulators.  An engine holds S shot slots of one model (S = 1 for the
 // one-shot-at-a-time path); every step kernel launch advances all active
-// slots.  The time loop is recorded once per geometry as HIP graphs of
+// slots.  Where the slots' tiles fit the chip the time loop is one launch
+// (ifos_resident.h); else it is recorded once per geometry as HIP graphs of
 // U = k*DTINV steps and replayed NT/U times; kernels read the step number
 // from a device counter so one graph serves every block of steps.
 #include <hip/hip_runtime.h>
@@ -216,6 +217,10 @@ struct ifos_engine {
     int resident_mode = -1;         // 1 wherever it fits, 0 never, -1 by rule (use_resident)
     bool loop_given = false;        // the caller chose a loop or launch shape of the per-step kernels
     bool resident_last = false;     // the last run took it
+    // runs to do with the per-step kernels before it is tried again, after one
+    // that was given up (another process may hold part of the GPU for long: each
+    // attempt would wait resident_limit); doubled each time, 1 after a success
+    int resident_skip = 0, resident_back = 1;
     int ncu = 0, lds_max = 0;
     unsigned long long *inbox = nullptr;
     size_t inbox_words = 0;
@@ -950,7 +955,7 @@ static ResidentPlan plan_of(const ifos_engine *E, int nslots)
 static bool use_resident(const ifos_engine *E)
 {
     if (E->resident_mode == 0) return false;
-    if (E->resident_mode < 0 && (E->graph_mode >= 0 || E->loop_given || E->fused)) return false;
+    if (E->resident_mode < 0 && (E->graph_mode >= 0 || E->loop_given || E->resident_skip > 0)) return false;
     return E->nslots > 0 && plan_of(E, E->nslots).rows > 0;
 }
 
@@ -1016,10 +1021,16 @@ static int run_steps(ifos_engine *E, int sw, bool snapshots)
         ResidentTurn turn(E->device);
         if (turn.mine) {
             ENG_TRY(run_resident(E, sw, snapshots, E->resident_last));
-            if (E->resident_last) return 0;
+            if (E->resident_last) {
+                E->resident_back = 1;
+                return 0;
+            }
+            E->resident_skip = E->resident_back + 1;  // this run counts
+            E->resident_back = std::min(2 * E->resident_back, 64);
             ENG_TRY(zero_run(E, sw, snapshots));
         }
     }
+    if (E->resident_skip > 0) E->resident_skip--;
     return run_loop(E, sw, snapshots);
 }
 
@@ -1707,6 +1718,8 @@ extern "C" int ifos_engine_set_resident(ifos_engine *E, int mode)
 {
     if (mode < -1 || mode > 1) return ifos_set_error("resident mode must be -1, 0 or 1"), -2;
     E->resident_mode = mode;
+    E->resident_skip = 0;
+    E->resident_back = 1;
     return 0;
 }
 

@@ -136,7 +136,8 @@ int  ifos_engine_get_graphs(ifos_engine *e, int *on);
  * set_work_order, set_velocity_rows, set_velocity_lds, set_fused).  Same bits
  * either way.  A workgroup that waits longer than set_resident_wait's seconds
  * (default 0.2, negative restores it) gives the run up, and it is repeated
- * with the per-step kernels.  get_resident reports whether the next run will
+ * with the per-step kernels; with mode -1 the next run (then 2, 4, ... 64 runs)
+ * goes straight to those.  get_resident reports whether the next run will
  * take it, and whether the last one did. */
 int  ifos_engine_set_resident(ifos_engine *e, int mode);
 int  ifos_engine_get_resident(ifos_engine *e, int *next, int *last);

@@ -79,6 +79,21 @@ def test_run_given_up_is_repeated(gpu_lib):
     want, _ = outputs(w, 0, eprecond=1)
     have, used = outputs(w, 1, eprecond=1, wait=0.0)
     assert not used and same_bits(want, have)
+    # by rule: given up, one run without it, tried again (given up, two without)
+    eng = ifos_amd.Engine(w.cfg)
+    eng.set_model(**w.start)
+    eng.set_shot(w.shots[0].srcpos, w.shots[0].recpos)
+    eng.set_resident_wait(0.0)
+    seen = []
+    for _ in range(6):
+        seen.append(eng.get_resident()[0])
+        eng.forward(snapshots=False)
+        assert not eng.get_resident()[1]
+    assert seen == [True, False, True, False, False, True]
+    eng.set_resident_wait(-1.0)
+    eng.set_resident(-1)
+    eng.forward(snapshots=False)
+    assert eng.get_resident() == (True, True)
 
 
 def test_which_runs_take_it(gpu_lib):
