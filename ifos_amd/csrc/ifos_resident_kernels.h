@@ -31,14 +31,18 @@ struct ResLds {
 // three alone when elastic), DT times the two buoyancies.
 constexpr int coefficients(int L) { return 3 * L + 5; }
 
-// How many of them, the first in that order, sit in LDS instead of registers:
-// none with one row per thread, else as many as fit beside the largest tile.
-// (With all of them in registers 36 values of every thread spilled to scratch on
-// 1024x512, L=2, FDORDER 8, and a step took 13.0 us instead of 10.6.)
+// How many of them, the first in that order, sit in LDS instead of registers.
+// With several rows per thread as many as fit beside the largest tile (with all
+// of them in registers 36 values of every thread spilled to scratch on 1024x512,
+// L=2, FDORDER 8, and a step took 13.0 us instead of 10.6).  With one row only
+// where the registers would spill: L=2, FDORDER 12, 1024x256 7.9 / 7.0 us a step,
+// FDORDER 8, 1024x128 5.0 / 4.8, L=3, FDORDER 8, 1024x256 5.8 / 5.5, FDORDER 4 5.3 /
+// 5.1; L=2, FDORDER 4 does not spill and a gradient's pair of steps of 301x151 went
+// from 8.7 to 8.8.
 template <int N, int L, int R>
 constexpr int lds_coefficients()
 {
-    if (R == 1) return 0;
+    if (R == 1) return N >= 4 && L >= 2 ? 3 * L + 3 : L >= 3 ? 3 * L : 0;
     const int n = ((163840 - 256) / 4 - ResLds<N, R>::planes) / ResLds<N, R>::plane;
     return n < 0 ? 0 : n < coefficients(L) ? n : coefficients(L);
 }
