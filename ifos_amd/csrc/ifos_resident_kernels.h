@@ -25,6 +25,8 @@ struct ResLds {
     static constexpr int surface = yprof + 10 * TH;
     static constexpr int planes = surface + 4 * kTileX;  // per-cell coefficients outside registers, [plane][row][64]
     static constexpr int plane = TH * kTileX;
+    // the FP64 reciprocals of the profiles are read as whole doubles
+    static_assert(xprof % 2 == 0 && yprof % 2 == 0, "FP64 profile values at odd floats");
 };
 
 // Coefficients of a cell: 2 d, e, dip per mechanism, 2 f, g, fipjp (the latter
@@ -285,7 +287,8 @@ __global__ __launch_bounds__(kResidentThreads) void k_resident(const ResidentArg
     const ArgPtr pa = cmem(ra.a);
     const auto &a = *pa;
     const auto &g = a.g;
-    extern __shared__ float lds[];
+    // aligned for the profiles' doubles: the array begins behind s_stop
+    extern __shared__ __attribute__((aligned(16))) float lds[];
     __shared__ int s_stop;  // half step in which a thread of this workgroup gave up, 0: none
     const int wg = (int)(blockIdx.x % 8) * ra.per + (int)blockIdx.x / 8;
     if ((int)blockIdx.x / 8 >= ra.per || wg >= ra.nwg) return;
