@@ -63,6 +63,15 @@ struct ResidentArgs {
     unsigned long long limit;  // longest wait for a neighbour, ticks of the 100 MHz clock
 };
 
+// Cell of the padded grid whose materials row r of a thread is given (c: the cell
+// of its row 0): its own, or, where that lies past the grid's last row or column,
+// cell (1, 1), which every grid has.  The last tile's rows can lie a tile's height
+// past the padding.
+__host__ __device__ inline unsigned material_cell(unsigned c, int r, int pitch, bool inside)
+{
+    return inside ? c + (unsigned)(r * pitch) : (unsigned)pitch + 1u;
+}
+
 // launch shape of a resident run, decided on the host (resident_plan)
 struct ResidentPlan {
     int rows = 0;            // rows per thread, 0: not eligible

@@ -379,7 +379,7 @@ __global__ __launch_bounds__(kResidentThreads) void k_resident(const ResidentArg
     }
 #pragma unroll
     for (int r = 0; r < R; r++) {
-        const unsigned ci = (live[r] ? c + r * P : P + 1u) * 4u;  // cell (1, 1): every grid has it
+        const unsigned ci = material_cell(c, r, P, live[r]) * 4u;
         const float bx_ = at(gmem(a.rip), ci), by_ = at(gmem(a.rjp), ci);
         if (r == 0) ripk = bx_, rjpk = by_;
         set_coef(r, cDtx, g.DT * bx_);
@@ -420,7 +420,7 @@ __global__ __launch_bounds__(kResidentThreads) void k_resident(const ResidentArg
             y = rjpk;
         } else {
             const auto &b = *afresh(pa);
-            const unsigned ci = (afresh(c) + r * b.g.pitch) * 4u;
+            const unsigned ci = material_cell(afresh(c), r, b.g.pitch, live[r]) * 4u;
             x = at(gmem(b.rip), ci);
             y = at(gmem(b.rjp), ci);
         }

@@ -38,3 +38,18 @@ def test_lds_arrays_begin_aligned(tmp_path):
     sizes = [size for name, size in kernel_metadata(tmp_path) if "k_resident" in name]
     assert len(sizes) > 60  # stencil orders x mechanisms x rows per thread
     assert all(size % 8 == 0 for size in sizes), sorted(set(sizes))
+
+
+def test_material_loads_stay_in_the_grid(tmp_path):
+    """Rows of cells past the grid's last row, which the lowest tiles hold, read
+    the materials of a cell that exists."""
+    exe = tmp_path / "bounds"
+    lib = os.path.dirname(B.LIB)
+    subprocess.run([B.HIPCC, "--offload-host-only", "-O1", "-std=c++17", "-I" + B.CSRC,
+                    "-I" + os.path.join(B.ROOT, "include"), "-x", "hip",
+                    os.path.join(B.ROOT, "tests", "c", "resident_bounds.cpp"), "-o", str(exe), "-L" + lib,
+                    "-lifos2d_hip", "-Wl,-rpath," + lib], check=True)
+    plans, outside, unguarded = map(int, subprocess.run([str(exe)], check=True, stdout=subprocess.PIPE,
+                                                        text=True).stdout.split())
+    assert plans > 200 and unguarded > 0  # some rows do lie past the padding
+    assert outside == 0
