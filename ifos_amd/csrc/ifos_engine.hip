@@ -959,30 +959,35 @@ static bool use_resident(const ifos_engine *E)
     return E->nslots > 0 && plan_of(E, E->nslots).rows > 0;
 }
 
-// One resident run at a time on a device: two that share the compute units
-// could each hold what the other waits for until both give up.  A run that
-// finds the device taken uses the per-step kernels.
-struct ResidentTurn {
-    static constexpr int kDevices = 64;
-    static std::atomic<bool> &taken(int device)
+// Time loops under way on a device, of all engines of the process.  A one-launch
+// run holds every compute unit from its start to its end, so the launches of
+// another engine's per-step kernels would wait for the gaps between such runs
+// (a 2000x800 loop of 13 ms beside endless 1200x600 runs took 669 ms), and beside
+// their succession it may not get its own compute units before it gives up.
+// Two one-launch runs could each hold what the other waits for.  So only a loop
+// that has the device to itself is one launch; a per-step loop that begins while
+// one is running waits for that one at most.
+struct DeviceLoops {
+    std::atomic<int> running{0};
+    static DeviceLoops &of(int device)
     {
-        static std::atomic<bool> t[kDevices];
-        return t[device];
+        static DeviceLoops all[64];
+        return all[std::min(std::max(device, 0), 63)];
     }
-    int device;
-    bool mine;
-    explicit ResidentTurn(int d) : device(d), mine(d >= 0 && d < kDevices && !taken(d).exchange(true)) {}
-    ~ResidentTurn()
-    {
-        if (mine) taken(device) = false;
-    }
+};
+
+struct LoopTurn {
+    DeviceLoops &d;
+    explicit LoopTurn(int device) : d(DeviceLoops::of(device)) { d.running++; }
+    ~LoopTurn() { d.running--; }
+    bool alone() const { return d.running == 1; }
 };
 
 // done: the run is complete; false: it was not taken, or given up (zero_run
 // must precede another attempt)
-static int run_resident(ifos_engine *E, int sw, bool snapshots, bool &done)
+static int run_resident(ifos_engine *E, int sw, bool snapshots, const LoopTurn &turn, bool &done, bool &given_up)
 {
-    done = false;
+    done = given_up = false;
     const ResidentPlan p = plan_of(E, E->nslots);
     const size_t need = (size_t)p.nwg * 2 * p.words;
     if (need > E->inbox_words) {
@@ -1003,28 +1008,31 @@ static int run_resident(ifos_engine *E, int sw, bool snapshots, bool &done)
     r.inbox = E->inbox;
     r.stop = E->ctl + 2;
     r.limit = E->resident_limit;
+    if (!turn.alone()) return 0;
     HIP_TRY(launch_resident(a, r, p, E->stream));
     int stop = 0;
     HIP_TRY(hipMemcpyAsync(&stop, E->ctl + 2, sizeof stop, hipMemcpyDeviceToHost, E->stream));
     HIP_TRY(hipStreamSynchronize(E->stream));
     done = stop == 0;
+    given_up = !done;
     if (done) E->last_set = 0;
     return 0;
 }
 
-// a forward (sw 0) or adjoint run of NT steps from a zero state
-static int run_steps(ifos_engine *E, int sw, bool snapshots)
+// a forward (sw 0) or adjoint run of NT steps from a zero state; turn: held by
+// the caller until the stream has finished
+static int run_steps(ifos_engine *E, int sw, bool snapshots, const LoopTurn &turn)
 {
     ENG_TRY(zero_run(E, sw, snapshots));
     E->resident_last = false;
-    if (use_resident(E)) {
-        ResidentTurn turn(E->device);
-        if (turn.mine) {
-            ENG_TRY(run_resident(E, sw, snapshots, E->resident_last));
-            if (E->resident_last) {
-                E->resident_back = 1;
-                return 0;
-            }
+    if (use_resident(E) && turn.alone()) {
+        bool given_up = false;
+        ENG_TRY(run_resident(E, sw, snapshots, turn, E->resident_last, given_up));
+        if (E->resident_last) {
+            E->resident_back = 1;
+            return 0;
+        }
+        if (given_up) {
             E->resident_skip = E->resident_back + 1;  // this run counts
             E->resident_back = std::min(2 * E->resident_back, 64);
             ENG_TRY(zero_run(E, sw, snapshots));
@@ -1077,7 +1085,8 @@ extern "C" int ifos_engine_forward(ifos_engine *E, int store_snapshots)
     if (store_snapshots) ENG_TRY(ensure_snapshots(E));
     E->snap_valid = false;
     E->slot_grad_valid = false;
-    ENG_TRY(run_steps(E, 0, store_snapshots != 0));
+    const LoopTurn turn(E->device);
+    ENG_TRY(run_steps(E, 0, store_snapshots != 0, turn));
     ENG_TRY(check_nan(E));
     E->snap_valid = store_snapshots != 0;
     return 0;
@@ -1516,7 +1525,8 @@ extern "C" int ifos_engine_adjoint(ifos_engine *E)
         return ifos_set_error("adjoint needs a forward run with snapshots on the current model and shot"), -2;
     if (!E->tiles || !E->model_set) return ifos_set_error("adjoint needs set_model and set_shot"), -2;
     E->slot_grad_valid = false;
-    ENG_TRY(run_steps(E, 1, false));
+    const LoopTurn turn(E->device);
+    ENG_TRY(run_steps(E, 1, false, turn));
     GradArgs ga;
     memset(&ga, 0, sizeof ga);
     if (E->ep_mode) ENG_TRY(energy_weights(E, ga));

@@ -1,0 +1,73 @@
+"""Engines of one process that run at the same moment on a device: a time loop
+is one launch (k_resident) only while no other engine's loop is under way, and
+the results do not depend on what runs beside them."""
+import threading
+import time
+
+import numpy as np
+import pytest
+
+import ifos_amd
+from ifos_amd import workloads
+
+pytestmark = pytest.mark.gpu
+
+
+def engine(NX, NY, NT, L=0, order=4):
+    w = workloads.small_case(seed=12, NX=NX, NY=NY, NT=NT, FW=8, DTINV=4, FDORDER=order, L=L, VELOCITY=1)
+    eng = ifos_amd.Engine(w.cfg)
+    eng.set_model(**w.start)
+    eng.set_shot(w.shots[0].srcpos, w.shots[0].recpos)
+    return eng
+
+
+def test_one_launch_only_with_the_device_to_itself(gpu_lib):
+    print("[overlap] a loop beside a longer one", flush=True)
+    long_, short = engine(1200, 700, 4000), engine(128, 96, 100)
+    long_.set_resident(0)
+    short.forward(snapshots=False)
+    assert short.get_resident()[1]
+    want = [np.array(x) for x in short.seismograms()]
+    begun = threading.Event()
+
+    def work():
+        begun.set()
+        long_.forward(snapshots=False)
+
+    t = threading.Thread(target=work)
+    t.start()
+    begun.wait()
+    time.sleep(0.02)  # the long loop takes over 0.1 s
+    short.forward(snapshots=False)
+    beside = t.is_alive()
+    taken = short.get_resident()[1]
+    t.join()
+    assert beside and not taken
+    for x, y in zip(want, short.seismograms()):
+        assert np.array_equal(x, y)
+    short.forward(snapshots=False)
+    assert short.get_resident()[1]
+
+
+def test_gradients_do_not_depend_on_what_runs_beside(gpu_lib):
+    print("[overlap] three engines, ten gradients each", flush=True)
+    engines = [engine(200, 90, 120, L=2, order=8), engine(400, 120, 80), engine(700, 300, 60, L=1)]
+    obs = [np.random.default_rng(4).standard_normal((2,) + e.seismograms()[0].shape).astype(np.float32) for e in engines]
+    want = []
+    for e, o in zip(engines, obs):
+        e.shot_gradient(o[0], o[1])
+        want.append(np.array(e.gradient()))
+    wrong = []
+
+    def work(e, o, ref):
+        for _ in range(10):
+            e.shot_gradient(o[0], o[1])
+            if not np.array_equal(np.array(e.gradient()).view(np.uint8), ref.view(np.uint8)):
+                wrong.append(e.cfg.NX)
+
+    threads = [threading.Thread(target=work, args=x) for x in zip(engines, obs, want)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
