@@ -945,18 +945,23 @@ static int zero_run(ifos_engine *E, int sw, bool snapshots)
 // ---------------------------------------------------------------------------
 // the time loop as one launch
 // ---------------------------------------------------------------------------
-static ResidentPlan plan_of(const ifos_engine *E, int nslots)
+static ResidentPlan plan_of(const ifos_engine *E, int sw, bool snapshots)
 {
-    return resident_plan(geom(E), E->c.L, nslots, E->snap_prec, E->ncu, (size_t)E->lds_max);
+    return resident_plan(geom(E), E->c.L, E->nslots, sw == 0 && snapshots ? E->snap_prec : 0, E->ncu,
+                         (size_t)E->lds_max);
 }
 
 // Taken wherever the shots' tiles fit the chip one per compute unit, unless
-// the caller chose a loop or launch shape of the per-step kernels.
-static bool use_resident(const ifos_engine *E)
+// the caller chose a loop or launch shape of the per-step kernels or those are
+// faster (resident_fill16).
+static bool use_resident(const ifos_engine *E, int sw, bool snapshots)
 {
-    if (E->resident_mode == 0) return false;
-    if (E->resident_mode < 0 && (E->graph_mode >= 0 || E->loop_given || E->resident_skip > 0)) return false;
-    return E->nslots > 0 && plan_of(E, E->nslots).rows > 0;
+    if (E->resident_mode == 0 || E->nslots < 1) return false;
+    const ResidentPlan p = plan_of(E, sw, snapshots);
+    if (E->resident_mode > 0 || !p.rows) return p.rows > 0;
+    if (E->graph_mode >= 0 || E->loop_given || E->resident_skip > 0) return false;
+    return !(sw == 0 && snapshots && E->snap_prec) ||
+           100 * p.cells >= resident_fill16(E->N, E->c.L, p.rows, E->c.DTINV) * kResidentThreads / kTileX * p.rows;
 }
 
 // Time loops under way on a device, of all engines of the process.  A one-launch
@@ -988,7 +993,7 @@ struct LoopTurn {
 static int run_resident(ifos_engine *E, int sw, bool snapshots, const LoopTurn &turn, bool &done, bool &given_up)
 {
     done = given_up = false;
-    const ResidentPlan p = plan_of(E, E->nslots);
+    const ResidentPlan p = plan_of(E, sw, snapshots);
     const size_t need = (size_t)p.nwg * 2 * p.words;
     if (need > E->inbox_words) {
         dfree(E->inbox);
@@ -1025,7 +1030,7 @@ static int run_steps(ifos_engine *E, int sw, bool snapshots, const LoopTurn &tur
 {
     ENG_TRY(zero_run(E, sw, snapshots));
     E->resident_last = false;
-    if (use_resident(E) && turn.alone()) {
+    if (use_resident(E, sw, snapshots) && turn.alone()) {
         bool given_up = false;
         ENG_TRY(run_resident(E, sw, snapshots, turn, E->resident_last, given_up));
         if (E->resident_last) {
@@ -1651,10 +1656,11 @@ extern "C" size_t ifos_engine_bytes(const ifos_config *c, int slots, int snap_pr
     StepGeom g{};
     g.NX = c->NX; g.NY = c->NY; g.N = N; g.FREE_SURF = c->FREE_SURF; g.BOUNDARY = c->BOUNDARY;
     size_t inbox = 0;
-    for (int s = 1; s <= std::min(slots, 256); s++) {
-        const ResidentPlan p = resident_plan(g, c->L, s, snap_prec, 256, 163840);
-        if (p.rows) inbox = std::max(inbox, sizeof(unsigned long long) * 2 * (size_t)p.nwg * p.words);
-    }
+    for (int s = 1; s <= std::min(slots, 256); s++)
+        for (int prec : {0, snap_prec}) {
+            const ResidentPlan p = resident_plan(g, c->L, s, prec, 256, 163840);
+            if (p.rows) inbox = std::max(inbox, sizeof(unsigned long long) * 2 * (size_t)p.nwg * p.words);
+        }
     b += inbox;
     return b;
 }
@@ -1735,7 +1741,7 @@ extern "C" int ifos_engine_set_resident(ifos_engine *E, int mode)
 
 extern "C" int ifos_engine_get_resident(ifos_engine *E, int *next, int *last)
 {
-    if (next) *next = use_resident(E) ? 1 : 0;
+    if (next) *next = use_resident(E, 0, E->snap_prec != 0) ? 1 : 0;
     if (last) *last = E->resident_last ? 1 : 0;
     return 0;
 }

@@ -44,6 +44,28 @@ constexpr bool resident_pays(int N, int L, int rows, int th)
     return !crowded || th >= 16 * rows - 8;
 }
 
+// A step that stores 16-bit snapshots costs more here than in the per-step kernels
+// (the values wait in memory for the scale of their tile, behind a barrier; tiles
+// round up to multiples of eight rows), so with three and more rows per thread such
+// a forward run has to fill more of the tile the more often it stores: this many
+// percent of the 16 * rows rows of cells, by the stencil's reach.  Forward runs, BF16,
+// how many times as fast as the per-step kernels at DTINV 1 and 8: elastic, FDORDER 8,
+// 82 of 96 rows of cells 0.74 and 1.15, 80 of 80 0.97 and 1.48; L=2, FDORDER 8, 50 of 64
+// 0.90 and 1.13, 48 of 48 1.32 and 1.91; L=3, FDORDER 12, 40 of 48 0.88 and 0.98, 48 of
+// 48 1.00 and 1.09.  With the 25 or 40 percent of every step's store the heights at
+// which the two are equal lie within 5 of the table at DTINV 1, 2, 3, 4, 6 and 8; one
+// and two rows are faster throughout.
+constexpr int resident_fill16(int N, int L, int rows, int DTINV)
+{
+    constexpr unsigned char share[9][6] = {
+        {46, 53, 58, 60, 60, 53}, {57, 65, 65, 60, 65, 67}, {51, 61, 62, 73, 75, 67}, {63, 78, 77, 84, 76, 84},  // L=0, 3-6
+        {44, 44, 44, 52, 45, 49}, {53, 51, 55, 73, 60, 69},                                                      // L=1, 3-4
+        {44, 44, 52, 63, 52, 68}, {66, 68, 76, 83, 83, 83},                                                      // L=2, 3-4
+        {44, 56, 71, 84, 79, 84}};                                                                               // L=3, 3
+    if (rows < 3) return 0;
+    return share[(L == 0 ? 0 : 2 + 2 * L) + rows - 3][N - 1] + (L == 0 && rows >= 5 ? 40 : 25) / DTINV;
+}
+
 constexpr int kWordsPerThread = 3;  // inbox words a thread polls, one row per thread
 
 // A line of the inbox is one word per cell: the value in the low half, the
@@ -76,11 +98,13 @@ __host__ __device__ inline unsigned material_cell(unsigned c, int r, int pitch, 
 struct ResidentPlan {
     int rows = 0;            // rows per thread, 0: not eligible
     int ty = 0, th = 0, tiles_y = 0, nwg = 0, words = 0;
+    int cells = 0;           // rows of cells a tile has to hold (th: rounded up)
     size_t lds = 0;
 };
 
 // the plan for nslots shots of a grid on a device of ncu compute units with
-// lds_max bytes of LDS per workgroup; rows 0 when the run does not fit
+// lds_max bytes of LDS per workgroup; snap_prec: that of the snapshots the run
+// stores, 0 when it stores none; rows 0 when the run does not fit
 ResidentPlan resident_plan(const StepGeom &g, int L, int nslots, int snap_prec, int ncu, size_t lds_max);
 // one run of NT steps, fields zero at the start; r: a, inbox, stop and limit set
 hipError_t launch_resident(const StepArgs &a, ResidentArgs r, const ResidentPlan &p, hipStream_t s);

@@ -144,10 +144,11 @@ ResidentPlan resident_plan(const StepGeom &g, int L, int nslots, int snap_prec, 
     while (line * (kTileX + th) > kWordsPerThread * kTileX * th) th++;
     for (int rows = 1; rows <= most; rows++) {
         int ty = (th + rows - 1) / rows;
-        // the scales of 16-bit snapshots belong to 64x8 tiles
+        // the scales of 16-bit snapshots belong to 64x8 tiles, which are formed whole
         while (snap_prec && ty * rows % kTileY) ty++;
         if (ty > kResidentThreads / kTileX) continue;
         p.ty = ty;
+        p.cells = th;
         p.th = ty * rows;
         p.tiles_y = (g.NY + p.th - 1) / p.th;
         p.nwg = nbx * p.tiles_y * nslots;

@@ -133,12 +133,15 @@ int  ifos_engine_get_graphs(ifos_engine *e, int *on);
  * half step.  mode 1 takes it wherever the shots' tiles fit the chip, 0
  * never, -1 (the default) wherever they fit unless the caller chose a loop or
  * a launch shape of the per-step kernels (set_graphs, set_launch,
- * set_work_order, set_velocity_rows, set_velocity_lds, set_fused).  Same bits
+ * set_work_order, set_velocity_rows, set_velocity_lds, set_fused), or those
+ * are faster (forward runs that store 16-bit snapshots every few steps on
+ * large tiles), or another engine's run is under way on the device.  Same bits
  * either way.  A workgroup that waits longer than set_resident_wait's seconds
  * (default 0.2, negative restores it) gives the run up, and it is repeated
  * with the per-step kernels; with mode -1 the next run (then 2, 4, ... 64 runs)
- * goes straight to those.  get_resident reports whether the next run will
- * take it, and whether the last one did. */
+ * goes straight to those.  get_resident reports whether the next forward
+ * run will take it (with 16-bit snapshot precision: one that stores snapshots)
+ * if the device is free, and whether the last run did. */
 int  ifos_engine_set_resident(ifos_engine *e, int mode);
 int  ifos_engine_get_resident(ifos_engine *e, int *next, int *last);
 int  ifos_engine_set_resident_wait(ifos_engine *e, double seconds);
