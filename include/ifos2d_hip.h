@@ -186,7 +186,8 @@ int  ifos_engine_get_fused(ifos_engine *e, int *on);
  * of each kernel), the two-kernel step and the one-kernel step
  * (ifos_engine_set_fused), keep the fastest, zero the stepped wavefields;
  * reports the pick (grid: the stress step's or the one kernel's) and its
- * time per step. */
+ * time per step.  Where a forward run is one launch (set_resident) the pick
+ * serves runs that find the device taken, and the time is the one launch's. */
 int  ifos_engine_autotune(ifos_engine *e, int reps, int *spb, int *grid, double *ms_per_step);
 /* Forward run (src/IFOS2D.c:1651-1894); snapshots every DTINV steps if asked. */
 int  ifos_engine_forward(ifos_engine *e, int store_snapshots);

@@ -1,5 +1,7 @@
 """The one-launch time loop with several rows of cells per thread: which runs
 take it."""
+import time
+
 import numpy as np
 import pytest
 
@@ -31,3 +33,26 @@ def test_16bit_snapshots_on_large_tiles(gpu_lib, NX, NY, L, order, DTINV, taken)
     assert eng.get_resident()[1] == plain
     eng.forward(snapshots=False)
     assert eng.get_resident()[1] == plain
+
+
+def test_autotuner_reports_the_run_that_follows(gpu_lib):
+    """The time per step is that of the one launch where runs take it: the
+    per-step kernels take more than twice as long on this grid."""
+    print("[resident] autotuner's time", flush=True)
+    w = workloads.small_case(seed=14, NX=400, NY=200, L=0, NT=1000, FW=10, DTINV=4, VELOCITY=1, FDORDER=4)
+    eng = ifos_amd.Engine(w.cfg)
+    eng.set_model(**w.start)
+    eng.set_shot(w.shots[0].srcpos, w.shots[0].recpos)
+    eng.forward(snapshots=False)
+    want = [np.array(x) for x in eng.seismograms()]
+    ms = eng.autotune(reps=3)[2]
+    took = []
+    for _ in range(5):
+        t0 = time.perf_counter()
+        eng.forward(snapshots=False)
+        took.append((time.perf_counter() - t0) * 1e3 / w.cfg.NT)
+    assert eng.get_resident()[1]
+    print(f"autotuner {ms * 1e3:.2f} us a step, run {min(took) * 1e3:.2f}", flush=True)
+    assert ms < 1.5 * min(took)
+    for x, y in zip(want, eng.seismograms()):
+        assert np.array_equal(x, y)
