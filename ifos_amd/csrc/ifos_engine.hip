@@ -383,7 +383,10 @@ static int engine_create(const ifos_config *cfg, int device, int slots, ifos_eng
     if (dmalloc(&E->explosive, sizeof(int) * slots) != hipSuccess) return fail(-3);
     hipMemsetAsync(E->explosive, 0, sizeof(int) * slots, E->stream);
     if (dmalloc(&E->dargs, sizeof(StepArgs) * 4) != hipSuccess) return fail(-3);
-    if (dmalloc(&E->point_map, sizeof(int) * 2 * E->plane * slots) != hipSuccess) return fail(-3);
+    if (dmalloc(&E->point_map, sizeof(int) * 2 * E->plane * slots) != hipSuccess) {
+        ifos_set_error("device allocation of the point maps of %d slots failed", slots);
+        return fail(-3);
+    }
     if (hipStreamSynchronize(E->stream) != hipSuccess) {
         ifos_set_error("engine set-up failed on the device");
         return fail(-1);
@@ -989,8 +992,9 @@ struct LoopTurn {
     bool alone() const { return d.running == 1; }
 };
 
-// done: the run is complete; false: it was not taken, or given up (zero_run
-// must precede another attempt)
+// done: the run is complete; false: it was not taken (memory or launch resources
+// ran short, or another engine came first), or given up (zero_run must precede
+// another attempt)
 static int run_resident(ifos_engine *E, int sw, bool snapshots, const LoopTurn &turn, bool &done, bool &given_up)
 {
     done = given_up = false;
@@ -1000,7 +1004,11 @@ static int run_resident(ifos_engine *E, int sw, bool snapshots, const LoopTurn &
         dfree(E->inbox);
         E->inbox = nullptr;
         E->inbox_words = 0;
-        HIP_TRY(dmalloc(&E->inbox, sizeof(unsigned long long) * need));
+        if (dmalloc(&E->inbox, sizeof(unsigned long long) * need) != hipSuccess) {
+            E->inbox = nullptr;
+            (void)hipGetLastError();  // the per-step kernels need no inbox
+            return 0;
+        }
         E->inbox_words = need;
     }
     StepArgs a = step_args(E, sw, snapshots);
@@ -1015,7 +1023,10 @@ static int run_resident(ifos_engine *E, int sw, bool snapshots, const LoopTurn &
     r.stop = E->ctl + 2;
     r.limit = E->resident_limit;
     if (!turn.alone()) return 0;
-    HIP_TRY(launch_resident(a, r, p, E->stream));
+    if (launch_resident(a, r, p, E->stream) != hipSuccess) {
+        (void)hipGetLastError();
+        return 0;
+    }
     int stop = 0;
     HIP_TRY(hipMemcpyAsync(&stop, E->ctl + 2, sizeof stop, hipMemcpyDeviceToHost, E->stream));
     HIP_TRY(hipStreamSynchronize(E->stream));
