@@ -218,10 +218,6 @@ struct ifos_engine {
     int resident_mode = -1;         // 1 wherever it fits, 0 never, -1 by rule (use_resident)
     bool loop_given = false;        // the caller chose a loop or launch shape of the per-step kernels
     bool resident_last = false;     // the last run took it
-    // runs to do with the per-step kernels before it is tried again, after one
-    // that was given up (another process may hold part of the GPU for long: each
-    // attempt would wait resident_limit); doubled each time, 1 after a success
-    int resident_skip = 0, resident_back = 1;
     int ncu = 0, lds_max = 0;
     unsigned long long *inbox = nullptr;
     size_t inbox_words = 0;
@@ -949,25 +945,6 @@ static int zero_run(ifos_engine *E, int sw, bool snapshots)
 // ---------------------------------------------------------------------------
 // the time loop as one launch
 // ---------------------------------------------------------------------------
-static ResidentPlan plan_of(const ifos_engine *E, int sw, bool snapshots)
-{
-    return resident_plan(geom(E), E->c.L, E->nslots, sw == 0 && snapshots ? E->snap_prec : 0, E->ncu,
-                         (size_t)E->lds_max);
-}
-
-// Taken wherever the shots' tiles fit the chip one per compute unit, unless
-// the caller chose a loop or launch shape of the per-step kernels or those are
-// faster (resident_fill16).
-static bool use_resident(const ifos_engine *E, int sw, bool snapshots)
-{
-    if (E->resident_mode == 0 || E->nslots < 1) return false;
-    const ResidentPlan p = plan_of(E, sw, snapshots);
-    if (E->resident_mode > 0 || !p.rows) return p.rows > 0;
-    if (E->graph_mode >= 0 || E->loop_given || E->resident_skip > 0) return false;
-    return !(sw == 0 && snapshots && E->snap_prec) ||
-           100 * p.cells >= resident_fill16(E->N, E->c.L, p.rows, E->c.DTINV) * kResidentThreads / kTileX * p.rows;
-}
-
 // Time loops under way on a device, of all engines of the process.  A one-launch
 // run holds every compute unit from its start to its end, so the launches of
 // another engine's per-step kernels would wait for the gaps between such runs
@@ -978,6 +955,11 @@ static bool use_resident(const ifos_engine *E, int sw, bool snapshots)
 // one is running waits for that one at most.
 struct DeviceLoops {
     std::atomic<int> running{0};
+    // runs to do with the per-step kernels before the one launch is tried again,
+    // after one that was given up (another process may hold part of the GPU for
+    // long: each attempt would wait resident_limit, each engine's first one too if
+    // it did not learn from the others'); doubled each time, 1 after a success
+    std::atomic<int> skip{0}, back{1};
     static DeviceLoops &of(int device)
     {
         static DeviceLoops all[64];
@@ -991,6 +973,31 @@ struct LoopTurn {
     ~LoopTurn() { d.running--; }
     bool alone() const { return d.running == 1; }
 };
+
+static ResidentPlan plan_of(const ifos_engine *E, int sw, bool snapshots)
+{
+    return resident_plan(geom(E), E->c.L, E->nslots, sw == 0 && snapshots ? E->snap_prec : 0, E->ncu,
+                         (size_t)E->lds_max);
+}
+
+// Taken wherever the shots' tiles fit the chip one per compute unit, unless
+// the caller chose a loop or launch shape of the per-step kernels or those are
+// faster (resident_fill16).
+static bool fits_resident(const ifos_engine *E, int sw, bool snapshots)
+{
+    if (E->resident_mode == 0 || E->nslots < 1) return false;
+    const ResidentPlan p = plan_of(E, sw, snapshots);
+    if (E->resident_mode > 0 || !p.rows) return p.rows > 0;
+    if (E->graph_mode >= 0 || E->loop_given) return false;
+    return !(sw == 0 && snapshots && E->snap_prec) ||
+           100 * p.cells >= resident_fill16(E->N, E->c.L, p.rows, E->c.DTINV) * kResidentThreads / kTileX * p.rows;
+}
+
+// ... and no run of the device was given up lately
+static bool use_resident(const ifos_engine *E, int sw, bool snapshots)
+{
+    return fits_resident(E, sw, snapshots) && (E->resident_mode > 0 || DeviceLoops::of(E->device).skip <= 0);
+}
 
 // done: the run is complete; false: it was not taken (memory or launch resources
 // ran short, or another engine came first), or given up (zero_run must precede
@@ -1042,20 +1049,24 @@ static int run_steps(ifos_engine *E, int sw, bool snapshots, const LoopTurn &tur
 {
     ENG_TRY(zero_run(E, sw, snapshots));
     E->resident_last = false;
-    if (use_resident(E, sw, snapshots) && turn.alone()) {
+    const bool fits = fits_resident(E, sw, snapshots), chosen = E->resident_mode > 0;
+    if (fits && !chosen && turn.d.skip > 0) {
+        turn.d.skip--;
+    } else if (fits && turn.alone()) {
         bool given_up = false;
         ENG_TRY(run_resident(E, sw, snapshots, turn, E->resident_last, given_up));
         if (E->resident_last) {
-            E->resident_back = 1;
+            turn.d.back = 1;
             return 0;
         }
         if (given_up) {
-            E->resident_skip = E->resident_back + 1;  // this run counts
-            E->resident_back = std::min(2 * E->resident_back, 64);
+            if (!chosen) {
+                turn.d.skip = turn.d.back.load();
+                turn.d.back = std::min(2 * turn.d.back, 64);
+            }
             ENG_TRY(zero_run(E, sw, snapshots));
         }
     }
-    if (E->resident_skip > 0) E->resident_skip--;
     return run_loop(E, sw, snapshots);
 }
 
@@ -1746,8 +1757,11 @@ extern "C" int ifos_engine_set_resident(ifos_engine *E, int mode)
 {
     if (mode < -1 || mode > 1) return ifos_set_error("resident mode must be -1, 0 or 1"), -2;
     E->resident_mode = mode;
-    E->resident_skip = 0;
-    E->resident_back = 1;
+    if (mode < 0) {  // try again at once
+        DeviceLoops &d = DeviceLoops::of(E->device);
+        d.skip = 0;
+        d.back = 1;
+    }
     return 0;
 }
 

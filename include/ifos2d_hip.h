@@ -139,7 +139,8 @@ int  ifos_engine_get_graphs(ifos_engine *e, int *on);
  * either way.  A workgroup that waits longer than set_resident_wait's seconds
  * (default 0.2, negative restores it) gives the run up, and it is repeated
  * with the per-step kernels; with mode -1 the next run (then 2, 4, ... 64 runs)
- * goes straight to those.  get_resident reports whether the next forward
+ * of the process on the device goes straight to those; setting mode -1 tries
+ * again at once.  get_resident reports whether the next forward
  * run will take it (with 16-bit snapshot precision: one that stores snapshots)
  * if the device is free, and whether the last run did. */
 int  ifos_engine_set_resident(ifos_engine *e, int mode);

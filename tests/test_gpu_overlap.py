@@ -71,3 +71,22 @@ def test_gradients_do_not_depend_on_what_runs_beside(gpu_lib):
     for t in threads:
         t.join()
     assert not wrong
+
+
+def test_a_run_given_up_holds_back_the_other_engines(gpu_lib):
+    """On a device that another process holds part of, every engine would wait
+    for itself before it turned to the per-step kernels."""
+    print("[overlap] a run given up", flush=True)
+    first, second = engine(200, 90, 40), engine(128, 96, 40)
+    first.set_resident(-1)
+    first.set_resident_wait(0.0)
+    first.forward(snapshots=False)
+    assert not first.get_resident()[1]
+    assert not second.get_resident()[0]
+    second.forward(snapshots=False)
+    assert not second.get_resident()[1]
+    second.forward(snapshots=False)  # tried again
+    assert second.get_resident() == (True, True)
+    first.set_resident_wait(-1.0)
+    first.forward(snapshots=False)
+    assert first.get_resident() == (True, True)
