@@ -156,10 +156,10 @@ struct ifos_engine {
     int nsrc = 0, ntr = 0, cap_src = 0, cap_tr = 0;
     std::vector<int> src_off, tr_off;
     int *explosive = nullptr;  // [slots] device
-    int *src_i = nullptr;   // ix, iy, type  [3][cap_src]
+    int *src_type = nullptr;  // [cap_src]
     double *src_d = nullptr;  // sin, cos [2][cap_src]
     float *sig = nullptr;   // [cap_src][NT]
-    int *rec_i = nullptr;   // rx, ry, kill [3][cap_tr]
+    int *kill = nullptr;    // [cap_tr]
     float *seis = nullptr;  // vx, vy, diff_vx, diff_vy, obs_vx, obs_vy: 6*[cap_tr][NT]
     double *trace_sums = nullptr;  // l2, en [2][cap_tr]
     std::vector<double> shot_misfit;  // l2, en per shot of the last residual
@@ -420,7 +420,7 @@ extern "C" void ifos_engine_destroy(ifos_engine *E)
     dfree(E->psi); dfree(E->ctl); dfree(E->explosive); dfree(E->dargs);
     dfree(E->wbuf); dfree(E->wbuf64); dfree(E->we_sum); dfree(E->ep_geom); dfree(E->we_max); dfree(E->red);
     dfree(E->tap_m); dfree(E->tap_ij); dfree(E->tap_lohi); dfree(E->tfbuf);
-    dfree(E->src_i); dfree(E->src_d); dfree(E->sig); dfree(E->rec_i); dfree(E->seis);
+    dfree(E->src_type); dfree(E->src_d); dfree(E->sig); dfree(E->kill); dfree(E->seis);
     dfree(E->trace_sums); dfree(E->snap); dfree(E->tiles); dfree(E->point_map);
     dfree(E->inbox);
     if (E->stream) hipStreamDestroy(E->stream);
@@ -568,19 +568,19 @@ extern "C" int ifos_engine_set_shots(ifos_engine *E, int nshots, const int *nsrc
     E->snap_valid = false;
     E->slot_grad_valid = false;
     if (nsrc > E->cap_src) {
-        dfree(E->src_i); dfree(E->src_d); dfree(E->sig);
-        E->src_i = nullptr; E->src_d = nullptr; E->sig = nullptr;
+        dfree(E->src_type); dfree(E->src_d); dfree(E->sig);
+        E->src_type = nullptr; E->src_d = nullptr; E->sig = nullptr;
         E->cap_src = nsrc;
-        HIP_TRY(dmalloc(&E->src_i, sizeof(int) * 3 * nsrc));
+        HIP_TRY(dmalloc(&E->src_type, sizeof(int) * nsrc));
         HIP_TRY(dmalloc(&E->src_d, sizeof(double) * 2 * nsrc));
         HIP_TRY(dmalloc(&E->sig, sizeof(float) * (size_t)nsrc * c.NT));
         drop_graphs(E);
     }
     if (ntr > E->cap_tr) {
-        dfree(E->rec_i); dfree(E->seis); dfree(E->trace_sums);
-        E->rec_i = nullptr; E->seis = nullptr; E->trace_sums = nullptr;
+        dfree(E->kill); dfree(E->seis); dfree(E->trace_sums);
+        E->kill = nullptr; E->seis = nullptr; E->trace_sums = nullptr;
         E->cap_tr = ntr;
-        HIP_TRY(dmalloc(&E->rec_i, sizeof(int) * 3 * ntr));
+        HIP_TRY(dmalloc(&E->kill, sizeof(int) * ntr));
         HIP_TRY(dmalloc(&E->seis, sizeof(float) * 6 * (size_t)ntr * c.NT));
         HIP_TRY(dmalloc(&E->trace_sums, sizeof(double) * 2 * ntr));
         HIP_TRY(hipMemsetAsync(E->seis, 0, sizeof(float) * 6 * (size_t)ntr * c.NT, E->stream));
@@ -608,35 +608,24 @@ extern "C" int ifos_engine_set_shots(ifos_engine *E, int nshots, const int *nsrc
     HIP_TRY(hipMemcpyAsync(E->explosive, expl.data(), sizeof(int) * nshots, hipMemcpyHostToDevice, E->stream));
     HIP_TRY(hipStreamSynchronize(E->stream));
     if (nsrc) {
-        std::vector<int> si(3 * (size_t)E->cap_src, 0);
+        std::vector<int> type(nsrc);
         std::vector<double> sd(2 * (size_t)E->cap_src, 0.0);
         for (int l = 0; l < nsrc; l++) {
             const float *sp = srcpos + (size_t)l * IFOS_SRC_STRIDE;
-            si[l] = (int)sp[0];
-            si[E->cap_src + l] = (int)sp[1];
-            si[2 * E->cap_src + l] = (int)sp[7];
+            type[l] = (int)sp[7];
             float azi_rad = sp[6] * 3.141592653589793 / 180;  // src/update_v_PML.c:556
             sd[l] = sin(azi_rad);
             sd[E->cap_src + l] = cos(azi_rad);
         }
         std::vector<float> w((size_t)nsrc * c.NT);
         ifos_wavelet(&c, nsrc, srcpos, w.data());
-        HIP_TRY(hipMemcpyAsync(E->src_i, si.data(), sizeof(int) * si.size(), hipMemcpyHostToDevice, E->stream));
+        HIP_TRY(hipMemcpyAsync(E->src_type, type.data(), sizeof(int) * nsrc, hipMemcpyHostToDevice, E->stream));
         HIP_TRY(hipMemcpyAsync(E->src_d, sd.data(), sizeof(double) * sd.size(), hipMemcpyHostToDevice, E->stream));
         HIP_TRY(hipMemcpyAsync(E->sig, w.data(), sizeof(float) * w.size(), hipMemcpyHostToDevice, E->stream));
         filter_traces(E, E->sig, nsrc, c.SOURCE_SHAPE != 6);
         HIP_TRY(hipStreamSynchronize(E->stream));
         E->sig_host.swap(w);
         E->sig_given = false;
-    }
-    if (ntr) {
-        std::vector<int> ri(3 * (size_t)E->cap_tr, 0);
-        for (int t = 0; t < ntr; t++) {
-            ri[t] = recpos[2 * t];
-            ri[E->cap_tr + t] = recpos[2 * t + 1];
-        }
-        HIP_TRY(hipMemcpyAsync(E->rec_i, ri.data(), sizeof(int) * ri.size(), hipMemcpyHostToDevice, E->stream));
-        HIP_TRY(hipStreamSynchronize(E->stream));
     }
     // sources and receivers by tile (running counts) and by cell (the first
     // point of each cell, and the chain of those at the same one, in order)
@@ -778,7 +767,7 @@ static StepArgs step_args(ifos_engine *E, int sw, bool snapshots)
     PointMap src;
     src.start = E->tiles + E->off_src_start; src.next = E->tiles + E->off_src_next;
     src.map = E->point_map;
-    src.type = E->src_i + 2 * E->cap_src;
+    src.type = E->src_type;
     src.sin_azi = E->src_d; src.cos_azi = E->src_d + E->cap_src;
     src.sig = E->sig; src.sig1 = E->sig;
     PointMap rec;
@@ -1179,8 +1168,8 @@ extern "C" int ifos_engine_residual(ifos_engine *E, const float *obs_vx, const f
     }
     const int *dkill = nullptr;
     if (c.TRKILL && kill) {
-        HIP_TRY(hipMemcpyAsync(E->rec_i + 2 * E->cap_tr, kill, sizeof(int) * ntr, hipMemcpyHostToDevice, E->stream));
-        dkill = E->rec_i + 2 * E->cap_tr;
+        HIP_TRY(hipMemcpyAsync(E->kill, kill, sizeof(int) * ntr, hipMemcpyHostToDevice, E->stream));
+        dkill = E->kill;
     }
     double l2 = 0.0, en = 0.0;
     std::vector<double> h(2 * (size_t)ntr);
@@ -1671,8 +1660,8 @@ extern "C" size_t ifos_engine_bytes(const ifos_config *c, int slots, int snap_pr
     b += sizeof(float) * (size_t)(7 * c->NY * fw2 + 6 * fw2 * c->NX) * slots;  // CPML memory
     b += sizeof(int) * 2 * plane * slots;                                 // cells of sources and receivers
     b += sizeof(float) * (size_t)6 * ntr_total * c->NT;                   // seismograms etc.
-    b += (sizeof(float) * c->NT + 3 * sizeof(int) + 2 * sizeof(double)) * (size_t)nsrc_total;
-    b += (3 * sizeof(int) + 2 * sizeof(double)) * (size_t)ntr_total;
+    b += (sizeof(float) * c->NT + sizeof(int) + 2 * sizeof(double)) * (size_t)nsrc_total;
+    b += (sizeof(int) + 2 * sizeof(double)) * (size_t)ntr_total;
     if (snapshots) b += snapshot_bytes(*c, snap_prec) * slots + 256;
     // inboxes of the one-launch time loop, at most one workgroup of the
     // tallest tile on each of 256 compute units
