@@ -428,7 +428,6 @@ extern "C" void ifos_engine_destroy(ifos_engine *E)
     delete E;
 }
 
-// copy an interior [NY][NX] host array into a padded device grid
 // Materials of a model, one thread per cell: what ifos_setup_materials forms on
 // the host, operand for operand (the same bits), from the uploaded grids.  The
 // neighbours past the last row and column are the first ones (the halo of a

@@ -44,7 +44,7 @@ __device__ __forceinline__ const IFOS_GAS T *gmem(const T *p)
 {
     return (const IFOS_GAS T *)p;
 }
-// read-only data of a launch (tile lists, CPML profiles, flags) through the
+// read-only data of a launch (point counts of the tiles, CPML profiles, flags) through the
 // constant address space: the compiler may keep such loads scalar and
 // schedule them freely, since nothing writes them while the kernel runs
 #define IFOS_CAS __attribute__((address_space(4)))

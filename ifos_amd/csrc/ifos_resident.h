@@ -31,7 +31,11 @@ constexpr int kResidentThreads = 1024;  // largest workgroup: 64 columns x 16 ro
 // 33.6 / 29.4; L=1, four 28.8 / 25.0; L=2, three 26.4 / 17.9, four 31.1 / 27.7;
 // L=3, three 28.1 / 25.5.  Four rows with L=2 spill too much beyond FDORDER 8
 // (FDORDER 12: 35.0 / 34.7, a gradient 77.1 / 78.3).
-constexpr int resident_max_rows(int N, int L) { return L == 0 ? 6 : L == 1 || (L == 2 && N <= 4) ? 4 : L <= 3 ? 3 : 0; }
+// Six rows of FDORDER 12 exceed the LDS.
+constexpr int resident_max_rows(int N, int L)
+{
+    return L == 0 ? (N <= 5 ? 6 : 5) : L == 1 || (L == 2 && N <= 4) ? 4 : L <= 3 ? 3 : 0;
+}
 
 // Where the registers spill most the tiles have to be nearly full: a tile just
 // over the height of one row fewer takes as long as a full one.  Elastic,

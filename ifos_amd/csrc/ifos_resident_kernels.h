@@ -883,6 +883,7 @@ template <int N, int L, int R>
 static size_t resident_lds_rows(int rows)
 {
     typedef ResLds<N, R> D;
+    static_assert(4 * D::planes + 256 <= 163840, "fields of the tallest tile exceed the LDS");
     if (rows == R) return sizeof(float) * (size_t)(D::planes + lds_coefficients<N, L, R>() * D::plane);
     if constexpr (R < resident_max_rows(N, L)) return resident_lds_rows<N, L, R + 1>(rows);
     return (size_t)-1;
