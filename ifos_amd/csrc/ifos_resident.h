@@ -3,7 +3,8 @@
 //
 // Each workgroup owns a tile of 64 columns x th rows for the whole run.  The
 // wavefields of the tile and the halo its stencils read sit in LDS, the
-// memory variables and materials in registers.  After each half step a
+// memory variables in registers, the update coefficients in registers with one
+// row of cells per thread, else in LDS as far as they fit.  After each half step a
 // workgroup hands the N edge lines its neighbours read to their inboxes in
 // device memory and waits for theirs; nothing else synchronises the tiles.
 //
@@ -12,11 +13,14 @@
 // 3.7 us a step: 1.7 update, 0.7 polling and unpacking, 0.8 sending, 0.3 waiting
 // for the write-through stores that the polling loads queue behind, 0.2 for
 // neighbours), so the loop keeps divisions, address arithmetic and anything rare
-// out of its registers and its path; with more rows the instructions issued.
+// out of its registers and its path.  With more rows vector instructions fill about
+// half of a SIMD's cycles (1024x768 elastic: 834 per wavefront and step, four
+// wavefronts a SIMD, 4 cycles each, of 26 k); LDS, the exchange and reloads of spilled
+// values take the rest.
 // The per-step kernels pay two launches a step, each with its ramp, drain and
 // cold loads.  Time per forward step, those and this (us): FDORDER 8, L=2:
-// 1024x256 13.2 / 5.6, 1024x512 20.2 / 10.6, 1024x768 26.4 / 17.5; elastic:
-// 1200x600 FDORDER 8 18.9 / 11.2, 1024x256 FDORDER 4 10.2 / 5.1.
+// 1024x256 12.7 / 5.9, 1024x512 18.7 / 9.7, 1024x768 25.2 / 17.8; elastic:
+// 1024x768 FDORDER 8 19.5 / 11.6, 1024x256 FDORDER 4 10.1 / 5.0.
 #pragma once
 #include "ifos_step.h"
 
@@ -27,24 +31,27 @@ constexpr int kResidentThreads = 1024;  // largest workgroup: 64 columns x 16 ro
 // Rows of cells per thread the kernel is compiled for, by the stencil reach and
 // the number of relaxation mechanisms (0: not compiled).  1024 threads share a
 // compute unit's registers, 128 each, and its LDS.  us per forward step of a full
-// chip, per-step kernels and this, FDORDER 8: elastic, four rows 25.9 / 15.5, six
-// 33.6 / 29.4; L=1, four 28.8 / 25.0; L=2, three 26.4 / 17.9, four 31.1 / 27.7;
-// L=3, three 28.1 / 25.5.  Four rows with L=2 spill too much beyond FDORDER 8
-// (FDORDER 12: 35.0 / 34.7, a gradient 77.1 / 78.3).
-// Six rows of FDORDER 12 exceed the LDS.
+// chip, per-step kernels and this, FDORDER 8: elastic, four rows 23.7 / 13.8, six
+// 32.9 / 27.7; L=1, four 27.6 / 21.8; L=2, three 25.3 / 17.8, four 30.0 / 26.7;
+// L=3, three 27.0 / 24.5.  Four rows with L=2 spill too much beyond FDORDER 8
+// (FDORDER 12, 56 rows of cells: 32.0 / 34.5, 64 34.2 / 33.0).  Six rows of FDORDER 12
+// exceed the LDS.
 constexpr int resident_max_rows(int N, int L)
 {
     return L == 0 ? (N <= 5 ? 6 : 5) : L == 1 || (L == 2 && N <= 4) ? 4 : L <= 3 ? 3 : 0;
 }
 
 // Where the registers spill most the tiles have to be nearly full: a tile just
-// over the height of one row fewer takes as long as a full one.  Elastic,
-// FDORDER 8, a gradient's pair of steps (us): 65 rows of cells 55.9 / 57.5, 72
-// 60.5 / 54.7; L=2, 49 rows 59.5 / 62.3, 56 64.3 / 61.3; L=3, 33 rows 48.6 / 49.8,
-// 40 55.4 / 53.2.
+// over the height of one row fewer takes as long as a full one.  FDORDER 8, a
+// gradient's pair of steps (us), per-step kernels and this: L=2, 49 rows of cells 57.8
+// / 59.0, 52 60.3 / 60.4, 56 63.8 / 59.0; L=3, 33 rows 48.4 / 46.7 (a forward step
+// 21.2 / 21.3, FDORDER 12 53.4 / 55.0), 40 55.0 / 51.5; elastic with a snapshot every
+// step, 82 rows, FP32 forward 36.5 / 37.5, BF16 adjoint 53.1 / 56.9, 88 rows 38.8 / 37.6
+// and 57.1 / 58.1.  Elastic tiles of five rows are faster from their lowest height on:
+// 65 rows 55.2 / 48.3, FDORDER 12 63.9 / 58.1.
 constexpr bool resident_pays(int N, int L, int rows, int th)
 {
-    const bool crowded = N >= 4 && rows >= (L == 0 ? 5 : L == 3 ? 3 : 4) && L != 1;
+    const bool crowded = N >= 4 && rows >= (L == 0 ? 6 : L == 3 ? 3 : 4) && L != 1;
     return !crowded || th >= 16 * rows - 8;
 }
 

@@ -36,11 +36,11 @@ constexpr int coefficients(int L) { return 3 * L + 5; }
 // How many of them, the first in that order, sit in LDS instead of registers.
 // With several rows per thread as many as fit beside the largest tile (with all
 // of them in registers 36 values of every thread spilled to scratch on 1024x512,
-// L=2, FDORDER 8, and a step took 13.0 us instead of 10.6).  With one row only
-// where the registers would spill: L=2, FDORDER 12, 1024x256 7.9 / 7.0 us a step,
-// FDORDER 8, 1024x128 5.0 / 4.8, L=3, FDORDER 8, 1024x256 5.8 / 5.5, FDORDER 4 5.3 /
-// 5.1; L=2, FDORDER 4 does not spill and a gradient's pair of steps of 301x151 went
-// from 8.7 to 8.8.
+// L=2, FDORDER 8, and a step took 13.0 us instead of 10.6, 9.7 since the array is
+// aligned).  With one row only where the registers would spill: L=2, FDORDER 12,
+// 1024x256 7.9 / 7.0 us a step, FDORDER 8, 1024x128 5.0 / 4.8, L=3, FDORDER 8, 1024x256
+// 5.8 / 5.5, FDORDER 4 5.3 / 5.1; L=2, FDORDER 4 does not spill and a gradient's pair
+// of steps of 301x151 went from 8.7 to 8.8.
 template <int N, int L, int R>
 constexpr int lds_coefficients()
 {
@@ -287,7 +287,8 @@ __global__ __launch_bounds__(kResidentThreads) void k_resident(const ResidentArg
     const ArgPtr pa = cmem(ra.a);
     const auto &a = *pa;
     const auto &g = a.g;
-    // aligned for the profiles' doubles: the array begins behind s_stop
+    // aligned for the profiles' doubles: the array begins behind s_stop (at byte 4 a
+    // shot gradient of 1700x350, L=2 took 62.6 ms instead of 58.1)
     extern __shared__ __attribute__((aligned(16))) float lds[];
     __shared__ int s_stop;  // half step in which a thread of this workgroup gave up, 0: none
     const int wg = (int)(blockIdx.x % 8) * ra.per + (int)blockIdx.x / 8;
