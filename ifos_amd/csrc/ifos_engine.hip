@@ -1927,6 +1927,7 @@ extern "C" int ifos_engine_time_kernel(ifos_engine *E, int kernel, int reps, dou
 {
     HIP_TRY(hipSetDevice(E->device));
     if (!E->tiles || !E->model_set) return ifos_set_error("time_kernel needs set_model and set_shot"), -2;
+    const LoopTurn turn(E->device);
     StepArgs a = shaped_args(step_args(E, 0, false), E->shape);
     a.base = nullptr;
     a.nan_flag = nullptr;
@@ -1977,6 +1978,7 @@ extern "C" int ifos_engine_autotune(ifos_engine *E, int reps, int *spb_out, int 
 {
     HIP_TRY(hipSetDevice(E->device));
     if (!E->tiles || !E->model_set) return ifos_set_error("autotune needs set_model and set_shots"), -2;
+    const LoopTurn turn(E->device);  // its launches are to be timed beside no one-launch run
     if (reps < 1) reps = 1;
     int ncu = 0;
     HIP_TRY(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, E->device));
@@ -2087,7 +2089,6 @@ extern "C" int ifos_engine_autotune(ifos_engine *E, int reps, int *spb_out, int 
     // where the runs are one launch the shape serves those that find the device
     // taken; the time reported is that of the run itself
     if (use_resident(E, 0, false)) {
-        const LoopTurn turn(E->device);
         double run = 1e30;
         for (int k = 0; k < 2; k++) {
             ENG_TRY(zero_run(E, 0, false));
