@@ -227,6 +227,7 @@ class Engine:
         _check(lib().ifos_engine_set_graphs(self.h, int(mode)))
 
     def get_graphs(self):
+        """Whether the per-step kernels would be replayed as graphs (a run may be one launch: get_resident)."""
         on = C.c_int()
         _check(lib().ifos_engine_get_graphs(self.h, C.byref(on)))
         return bool(on.value)
@@ -236,7 +237,7 @@ class Engine:
         _check(lib().ifos_engine_set_resident(self.h, int(mode)))
 
     def get_resident(self):
-        """(the next run will take it, the last run did)."""
+        """(the next forward run will take it if the device is free, the last run did)."""
         a, b = C.c_int(), C.c_int()
         _check(lib().ifos_engine_get_resident(self.h, C.byref(a), C.byref(b)))
         return bool(a.value), bool(b.value)

@@ -125,24 +125,27 @@ int  ifos_engine_shot_misfit(ifos_engine *e, double *per_shot);
  * graphs below 2^19 cells x slots, where launching would be the bottleneck.
  * Results are the same bits either way.  The environment variable
  * IFOS_NO_GRAPH=1 (or 0) sets 0 (or 1) at creation.  get_graphs reports
- * what the next run will use. */
+ * what the next run of the per-step kernels will use; whether the run is one
+ * launch instead, get_resident says. */
 int  ifos_engine_set_graphs(ifos_engine *e, int mode);
 int  ifos_engine_get_graphs(ifos_engine *e, int *on);
 /* The whole time loop as one launch: each compute unit keeps a tile of the
  * grid for the run and exchanges edge lines with its neighbours' after every
  * half step.  mode 1 takes it wherever the shots' tiles fit the chip, 0
- * never, -1 (the default) wherever they fit unless the caller chose a loop or
- * a launch shape of the per-step kernels (set_graphs, set_launch,
- * set_work_order, set_velocity_rows, set_velocity_lds, set_fused), or those
- * are faster (forward runs that store 16-bit snapshots every few steps on
- * large tiles), or another engine's run is under way on the device.  Same bits
- * either way.  A workgroup that waits longer than set_resident_wait's seconds
- * (default 0.2, negative restores it) gives the run up, and it is repeated
- * with the per-step kernels; with mode -1 the next run (then 2, 4, ... 64 runs)
- * of the process on the device goes straight to those; setting mode -1 tries
- * again at once.  get_resident reports whether the next forward
- * run will take it (with 16-bit snapshot precision: one that stores snapshots)
- * if the device is free, and whether the last run did. */
+ * never, -1 (the default) wherever they fit unless
+ *   - the caller chose a loop or a launch shape of the per-step kernels
+ *     (set_graphs, until set_graphs(-1); set_launch, set_work_order,
+ *     set_velocity_rows, set_velocity_lds, set_fused, for the engine's life),
+ *   - or those are faster: forward runs that store 16-bit snapshots every few
+ *     steps on large tiles.
+ * In either mode a run beside another engine's forward or adjoint run on the
+ * device uses the per-step kernels.  Same bits every way.  A workgroup that waits
+ * longer than set_resident_wait's seconds (default 0.2, negative restores it)
+ * gives the run up, and it is repeated with the per-step kernels; with mode -1
+ * the next run (then 2, 4, ... 64 runs) of the process on the device goes straight
+ * to those; setting mode -1 tries again at once.  get_resident reports whether
+ * the next forward run will take it (with 16-bit snapshot precision: one that
+ * stores snapshots) if the device is free, and whether the last run did. */
 int  ifos_engine_set_resident(ifos_engine *e, int mode);
 int  ifos_engine_get_resident(ifos_engine *e, int *next, int *last);
 int  ifos_engine_set_resident_wait(ifos_engine *e, double seconds);

@@ -74,6 +74,7 @@ ROWS = [
     dict(R=4, NX=500, NY=1000, shots=2, L=1, FDORDER=12, VELOCITY=0, ep=3, ep64=1),
     dict(R=4, NX=1024, NY=900, L=0, FDORDER=10, snap="fp16", DTINV=1, FREE_SURF=0),
     dict(R=5, NX=1024, NY=1270, L=0, FDORDER=12, ep=1, ep64=1, FREE_SURF=0),
+    dict(R=5, NX=1024, NY=1034, L=0, FDORDER=8, FREE_SURF=0),
     dict(R=5, NX=500, NY=1250, shots=2, L=0, FDORDER=8, VELOCITY=0, snap="bf16", ep=1),
     dict(R=6, NX=1024, NY=1530, L=0, FDORDER=8, snap="fp16", ep=1, FREE_SURF=0),
     dict(R=6, NX=500, NY=1500, shots=2, L=0, FDORDER=4, VELOCITY=0, ep=3, DTINV=1),
