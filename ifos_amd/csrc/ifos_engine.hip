@@ -10,8 +10,13 @@
 // from a device counter so one graph serves every block of steps.
 #include <hip/hip_runtime.h>
 
+#include <fcntl.h>
+#include <sys/file.h>
+#include <unistd.h>
+
 #include <algorithm>
 #include <atomic>
+#include <cctype>
 #include <chrono>
 #include <cmath>
 #include <cstdarg>
@@ -933,33 +938,107 @@ static int zero_run(ifos_engine *E, int sw, bool snapshots)
 // ---------------------------------------------------------------------------
 // the time loop as one launch
 // ---------------------------------------------------------------------------
-// Time loops under way on a device, of all engines of the process.  A one-launch
-// run holds every compute unit from its start to its end, so the launches of
-// another engine's per-step kernels would wait for the gaps between such runs
-// (a 2000x800 loop of 13 ms beside endless 1200x600 runs took 669 ms), and beside
-// their succession it may not get its own compute units before it gives up.
-// Two one-launch runs could each hold what the other waits for.  So only a loop
-// that has the device to itself is one launch; a per-step loop that begins while
-// one is running waits for that one at most.
+// Time loops under way on a device.  A one-launch run holds every compute unit
+// from its start to its end, so the launches of another engine's per-step kernels
+// would wait for the gaps between such runs (a 2000x800 loop of 13 ms beside endless
+// 1200x600 runs took 669 ms, in another process 627), and beside their succession it
+// may not get its own compute units before it gives up.  Two one-launch runs could
+// each hold what the other waits for.  So only a loop that has the device to itself
+// is one launch; a loop that begins while one is running waits for that one at most.
+// Loops of one process count each other here; processes lock the device's directory
+// under /sys/bus/pci/devices (nothing is written): shared around per-step loops,
+// exclusively around a one-launch run.  A process waits for that lock with the one of
+// a file in the directory in hand, so that another cannot take it again and again
+// (without, two processes of 1200x600 runs of 6 ms waited up to 1 s for each other).
+// Where there is no such directory only the loops of the process are seen.
 struct DeviceLoops {
-    std::atomic<int> running{0};
+    std::mutex mu;                // of the changes of running and held
+    std::atomic<int> running{0}, held{LOCK_UN};
+    int dir = -1, queue = -1;
+    bool looked = false;
     // runs to do with the per-step kernels before the one launch is tried again,
-    // after one that was given up (another process may hold part of the GPU for
-    // long: each attempt would wait resident_limit, each engine's first one too if
-    // it did not learn from the others'); doubled each time, 1 after a success
+    // after one that was given up (something may hold part of the GPU for long: each
+    // attempt would wait resident_limit, each engine's first one too if it did not
+    // learn from the others'); doubled each time, 1 after a success
     std::atomic<int> skip{0}, back{1};
     static DeviceLoops &of(int device)
     {
         static DeviceLoops all[64];
         return all[std::min(std::max(device, 0), 63)];
     }
+    void look(int device)
+    {
+        if (looked) return;
+        looked = true;
+        char id[64] = "", path[128];
+        if (hipDeviceGetPCIBusId(id, sizeof id, device) != hipSuccess) {
+            (void)hipGetLastError();
+            return;
+        }
+        for (char *c = id; *c; c++) *c = (char)tolower(*c);
+        snprintf(path, sizeof path, "/sys/bus/pci/devices/%s", id);
+        dir = open(path, O_RDONLY | O_DIRECTORY | O_CLOEXEC);
+        if (dir < 0) return;
+        queue = openat(dir, "vendor", O_RDONLY | O_CLOEXEC);
+        if (queue >= 0) return;
+        close(dir);
+        dir = -1;
+    }
+    bool lock(int how)
+    {
+        // (a conversion that fails has dropped what was held)
+        held = flock(dir, how | LOCK_NB) == 0 ? how : LOCK_UN;
+        return held == how;
+    }
+    // exclusive if wanted and no other process has a loop under way, else shared,
+    // after another one's one-launch run; past 0.25 s neither
+    void acquire(bool exclusive)
+    {
+        if (dir < 0) return;
+        const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(250);
+        auto wait = [&]() {
+            if (std::chrono::steady_clock::now() > until) return false;
+            usleep(20);
+            return true;
+        };
+        while (flock(queue, LOCK_EX | LOCK_NB) != 0)
+            if (!wait()) return;
+        while (!(exclusive && lock(LOCK_EX)) && !lock(LOCK_SH))
+            if (!wait()) break;
+        flock(queue, LOCK_UN);
+    }
 };
 
 struct LoopTurn {
     DeviceLoops &d;
-    explicit LoopTurn(int device) : d(DeviceLoops::of(device)) { d.running++; }
-    ~LoopTurn() { d.running--; }
-    bool alone() const { return d.running == 1; }
+    LoopTurn(int device, bool one_launch) : d(DeviceLoops::of(device))
+    {
+        std::lock_guard<std::mutex> g(d.mu);
+        d.look(device);
+        if (d.running == 0) d.acquire(one_launch);
+        d.running++;
+    }
+    ~LoopTurn()
+    {
+        std::lock_guard<std::mutex> g(d.mu);
+        if (--d.running > 0) let_in();
+        else if (d.held != LOCK_UN) d.lock(LOCK_UN);
+    }
+    LoopTurn(const LoopTurn &) = delete;
+    // no other loop is under way, and none of another process will begin
+    bool alone() const { return d.running == 1 && (d.dir < 0 || d.held == LOCK_EX); }
+    // the loops of other processes may begin
+    void share()
+    {
+        std::lock_guard<std::mutex> g(d.mu);
+        let_in();
+    }
+
+private:
+    void let_in()
+    {
+        if (d.held == LOCK_EX) d.lock(LOCK_SH);
+    }
 };
 
 static ResidentPlan plan_of(const ifos_engine *E, int sw, bool snapshots)
@@ -1033,7 +1112,7 @@ static int run_resident(ifos_engine *E, int sw, bool snapshots, const LoopTurn &
 
 // a forward (sw 0) or adjoint run of NT steps from a zero state; turn: held by
 // the caller until the stream has finished
-static int run_steps(ifos_engine *E, int sw, bool snapshots, const LoopTurn &turn)
+static int run_steps(ifos_engine *E, int sw, bool snapshots, LoopTurn &turn)
 {
     ENG_TRY(zero_run(E, sw, snapshots));
     E->resident_last = false;
@@ -1055,6 +1134,7 @@ static int run_steps(ifos_engine *E, int sw, bool snapshots, const LoopTurn &tur
             ENG_TRY(zero_run(E, sw, snapshots));
         }
     }
+    turn.share();
     return run_loop(E, sw, snapshots);
 }
 
@@ -1101,7 +1181,7 @@ extern "C" int ifos_engine_forward(ifos_engine *E, int store_snapshots)
     if (store_snapshots) ENG_TRY(ensure_snapshots(E));
     E->snap_valid = false;
     E->slot_grad_valid = false;
-    const LoopTurn turn(E->device);
+    LoopTurn turn(E->device, use_resident(E, 0, store_snapshots != 0));
     ENG_TRY(run_steps(E, 0, store_snapshots != 0, turn));
     ENG_TRY(check_nan(E));
     E->snap_valid = store_snapshots != 0;
@@ -1541,7 +1621,7 @@ extern "C" int ifos_engine_adjoint(ifos_engine *E)
         return ifos_set_error("adjoint needs a forward run with snapshots on the current model and shot"), -2;
     if (!E->tiles || !E->model_set) return ifos_set_error("adjoint needs set_model and set_shot"), -2;
     E->slot_grad_valid = false;
-    const LoopTurn turn(E->device);
+    LoopTurn turn(E->device, use_resident(E, 1, false));
     ENG_TRY(run_steps(E, 1, false, turn));
     GradArgs ga;
     memset(&ga, 0, sizeof ga);
@@ -1927,7 +2007,7 @@ extern "C" int ifos_engine_time_kernel(ifos_engine *E, int kernel, int reps, dou
 {
     HIP_TRY(hipSetDevice(E->device));
     if (!E->tiles || !E->model_set) return ifos_set_error("time_kernel needs set_model and set_shot"), -2;
-    const LoopTurn turn(E->device);
+    const LoopTurn turn(E->device, false);
     StepArgs a = shaped_args(step_args(E, 0, false), E->shape);
     a.base = nullptr;
     a.nan_flag = nullptr;
@@ -1978,7 +2058,7 @@ extern "C" int ifos_engine_autotune(ifos_engine *E, int reps, int *spb_out, int 
 {
     HIP_TRY(hipSetDevice(E->device));
     if (!E->tiles || !E->model_set) return ifos_set_error("autotune needs set_model and set_shots"), -2;
-    const LoopTurn turn(E->device);  // its launches are to be timed beside no one-launch run
+    const LoopTurn turn(E->device, use_resident(E, 0, false));  // no one-launch run beside what is timed
     if (reps < 1) reps = 1;
     int ncu = 0;
     HIP_TRY(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, E->device));

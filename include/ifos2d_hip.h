@@ -139,7 +139,8 @@ int  ifos_engine_get_graphs(ifos_engine *e, int *on);
  *   - or those are faster: forward runs that store 16-bit snapshots every few
  *     steps on large tiles.
  * In either mode a run beside another engine's forward or adjoint run on the
- * device uses the per-step kernels.  Same bits every way.  A workgroup that waits
+ * device uses the per-step kernels, and a run waits up to 0.25 s for another
+ * process's one-launch run to end.  Same bits every way.  A workgroup that waits
  * longer than set_resident_wait's seconds (default 0.2, negative restores it)
  * gives the run up, and it is repeated with the per-step kernels; with mode -1
  * the next run (then 2, 4, ... 64 runs) of the process on the device goes straight

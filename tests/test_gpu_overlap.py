@@ -1,6 +1,9 @@
-"""Engines of one process that run at the same moment on a device: a time loop
-is one launch (k_resident) only while no other engine's loop is under way, and
-the results do not depend on what runs beside them."""
+"""Engines of one process, and of several, that run at the same moment on a
+device: a time loop is one launch (k_resident) only while no other engine's loop
+is under way, and the results do not depend on what runs beside them."""
+import ctypes as C
+import fcntl
+import os
 import threading
 import time
 
@@ -90,3 +93,46 @@ def test_a_run_given_up_holds_back_the_other_engines(gpu_lib):
     first.set_resident_wait(-1.0)
     first.forward(snapshots=False)
     assert first.get_resident() == (True, True)
+
+
+def test_other_processes_loops(gpu_lib):
+    """Processes lock the device's directory, shared around per-step loops and
+    exclusively around a one-launch run.  (Two descriptors of one process exclude
+    each other like those of two.)"""
+    print("[overlap] other processes", flush=True)
+    name = C.create_string_buffer(64)
+    assert gpu_lib.hipDeviceGetPCIBusId(name, 64, 0) == 0
+    path = "/sys/bus/pci/devices/" + name.value.decode().lower()
+    if not os.path.isdir(path):
+        pytest.skip("no directory of the device to lock")
+    eng = engine(200, 90, 40)
+    eng.set_resident(-1)
+    eng.forward(snapshots=False)
+    assert eng.get_resident()[1]
+    want = [np.array(x) for x in eng.seismograms()]
+
+    def run():
+        t0 = time.perf_counter()
+        eng.forward(snapshots=False)
+        for x, y in zip(want, eng.seismograms()):
+            assert np.array_equal(x, y)
+        return eng.get_resident()[1], time.perf_counter() - t0
+
+    other = os.open(path, os.O_RDONLY)
+    try:
+        fcntl.flock(other, fcntl.LOCK_SH)  # a per-step loop elsewhere
+        taken, took = run()
+        assert not taken and took < 0.2
+        fcntl.flock(other, fcntl.LOCK_UN)
+        assert run()[0]
+        fcntl.flock(other, fcntl.LOCK_EX)  # a one-launch run elsewhere: waited for
+        threading.Timer(0.05, lambda: fcntl.flock(other, fcntl.LOCK_UN)).start()
+        taken, took = run()
+        assert taken and 0.03 < took < 0.2
+        fcntl.flock(other, fcntl.LOCK_EX)  # one that does not end: not for ever
+        taken, took = run()
+        assert not taken and 0.2 < took < 1.0
+    finally:
+        os.close(other)
+    assert run()[0]
+    assert eng.get_resident()[0]
