@@ -17,6 +17,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cctype>
+#include <cerrno>
 #include <chrono>
 #include <cmath>
 #include <cstdarg>
@@ -950,7 +951,8 @@ static int zero_run(ifos_engine *E, int sw, bool snapshots)
 // exclusively around a one-launch run.  A process waits for that lock with the one of
 // a file in the directory in hand, so that another cannot take it again and again
 // (without, two processes of 1200x600 runs of 6 ms waited up to 1 s for each other).
-// Where there is no such directory only the loops of the process are seen.
+// Where there is no such directory, or no locks on it, only the process's own loops
+// are seen.
 struct DeviceLoops {
     std::mutex mu;                // of the changes of running and held
     std::atomic<int> running{0}, held{LOCK_UN};
@@ -980,9 +982,16 @@ struct DeviceLoops {
         dir = open(path, O_RDONLY | O_DIRECTORY | O_CLOEXEC);
         if (dir < 0) return;
         queue = openat(dir, "vendor", O_RDONLY | O_CLOEXEC);
-        if (queue >= 0) return;
+        if (queue >= 0 && lockable(queue) && lockable(dir)) return;
+        if (queue >= 0) close(queue);
         close(dir);
-        dir = -1;
+        dir = queue = -1;
+    }
+    // whether this file system has such locks (one that another process holds will do)
+    static bool lockable(int fd)
+    {
+        if (flock(fd, LOCK_SH | LOCK_NB) == 0) return flock(fd, LOCK_UN) == 0;
+        return errno == EWOULDBLOCK;
     }
     bool lock(int how)
     {
@@ -991,21 +1000,28 @@ struct DeviceLoops {
         return held == how;
     }
     // exclusive if wanted and no other process has a loop under way, else shared,
-    // after another one's one-launch run; past 0.25 s neither
+    // after another one's one-launch run; past 0.25 s neither, and the next wait is
+    // half as long, to 1 ms (a process that was stopped may hold the lock for ever)
+    int patience = 250;
     void acquire(bool exclusive)
     {
         if (dir < 0) return;
-        const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(250);
+        const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(patience);
         auto wait = [&]() {
             if (std::chrono::steady_clock::now() > until) return false;
             usleep(20);
             return true;
         };
-        while (flock(queue, LOCK_EX | LOCK_NB) != 0)
-            if (!wait()) return;
-        while (!(exclusive && lock(LOCK_EX)) && !lock(LOCK_SH))
-            if (!wait()) break;
-        flock(queue, LOCK_UN);
+        bool turn = true;
+        while (turn && flock(queue, LOCK_EX | LOCK_NB) != 0) turn = wait();
+        if (turn) {
+            // (once more exclusively where a one-launch run has just ended)
+            while (turn && !(exclusive && lock(LOCK_EX)) &&
+                   !(lock(LOCK_SH) && (!exclusive || lock(LOCK_EX) || lock(LOCK_SH))))
+                turn = wait();
+            flock(queue, LOCK_UN);
+        }
+        patience = turn ? 250 : std::max(patience / 2, 1);
     }
 };
 
